@@ -218,7 +218,7 @@ const std::array<AcrossLaunch64, kMaxAcross64>& across64_tab(); // index LA-1
 // ---- launchers of the remaining kernels (k_misc.hip)
 void launch_queue(const QueueArgs& a, int grid, hipStream_t st);
 void launch_reset_counter(uint32_t* c, hipStream_t st);
-void launch_vexpr(const VExprArgsT<float>& a, int64_t nwg, hipStream_t st);
-void launch_vexpr(const VExprArgsT<double>& a, int64_t nwg, hipStream_t st);
+void launch_vexpr(const VExprArgsT<float>& a, hipStream_t st);
+void launch_vexpr(const VExprArgsT<double>& a, hipStream_t st);
 
 } // namespace pcxd

@@ -1900,10 +1900,7 @@ int vexpr_eval(const S* srcs, int32_t nsrc, const I* prog, int32_t nprog, T* dst
     a.n      = n;
     if (n == 0)
         return PCX_SUCCESS;
-    int64_t nwg = (n + 255) / 256;
-    if (nwg > 16384)
-        nwg = 16384;
-    launch_vexpr(a, nwg, (hipStream_t)stream);
+    launch_vexpr(a, (hipStream_t)stream);
     HIPCHK(hipGetLastError());
     return PCX_SUCCESS;
 }

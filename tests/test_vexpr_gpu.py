@@ -193,3 +193,51 @@ def test_repack_double_bit_exact(orc, pa, sp, dp):
     assert np.array_equal(dst.to_complex(), z)
     with pytest.raises(pa.PcxError):
         pa.repack(dst, pa.vector(n, sp))  # float and double do not mix
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("pack", [1, 2, 4, 8])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_groups_remainders_and_alignment(pa, dtype, pack, shift):
+    """Expressions in groups of 16 bytes: sizes around a group, more sources than are loaded ahead,
+    operands in either stack order, vectors off 16-byte alignment (shift), and a program that is no
+    stack program.  Small integers, so every result is exact."""
+    import torch
+
+    from packed_amd import _lib
+
+    rng = np.random.default_rng(pack + 10 * shift)
+    for n in (1, 2, 3, 4, 5, 7, 8, 9, 255, 1023, 1030):
+        vals, vecs = [], []
+        for k in range(6):
+            z = (rng.integers(-8, 9, n) + 1j * rng.integers(-8, 9, n)).astype(np.complex128)
+            v = pa.vector.from_complex(z, (pack, 8)[k % 2], dtype=dtype)
+            room = torch.zeros(v.data.numel() + shift, dtype=v.data.dtype, device="cuda")
+            room[shift:] = v.data
+            vals.append(z)
+            vecs.append(pa.vector(n, v.pack, room[shift:], dtype))
+        a, b, c, d, e, f = vecs
+        x = vals
+
+        def out():
+            room = torch.full((pa.real_size(n, pack) + shift + 8,), 77.0, dtype=a.data.dtype, device="cuda")
+            return room, pa.vector(n, pack, room[shift:shift + pa.real_size(n, pack)], dtype)
+
+        cases = [(a * pa.conj(b) + c, x[0] * np.conj(x[1]) + x[2]),
+                 (a - (b * c - d * e), x[0] - (x[1] * x[2] - x[3] * x[4])),
+                 (2 - (a + b * (c - f)) * (1 + 2j) + e + d, 2 - (x[0] + x[1] * (x[2] - x[5])) * (1 + 2j) + x[4] + x[3]),
+                 (a * a, x[0] * x[0])]
+        for expr, want in cases:
+            room, dst = out()
+            pa.store(expr, dst)
+            assert np.array_equal(dst.to_complex(), want), (n, pack, shift)
+            assert torch.all(room[shift + pa.real_size(n, pack):] == 77.0)
+        # registers 2 and 0, loaded out of stack order: the register machine
+        room, dst = out()
+        VS, VI, ev = ((_lib.VSource64, _lib.VInstr64, _lib.lib().pcx_vexpr_eval_f64) if dtype == "float64"
+                      else (_lib.VSource, _lib.VInstr, _lib.lib().pcx_vexpr_eval))
+        srcs = (VS * 2)(VS(a.data_ptr(), a.pack), VS(b.data_ptr(), b.pack))
+        prog = (VI * 3)(VI(_lib.VOP["LOAD"], 2, 0, 0, 0, 0), VI(_lib.VOP["LOAD"], 0, 1, 0, 0, 0),
+                        VI(_lib.VOP["SUB"], 0, 2, 0, 0, 0))
+        _lib.check(ev(srcs, 2, prog, 3, dst.data_ptr(), pack, n, torch.cuda.current_stream().cuda_stream))
+        assert np.array_equal(dst.to_complex(), x[0] - x[1])
