@@ -11,6 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <array>
 #include <cstdint>
 #include <utility>
@@ -33,6 +34,7 @@ using ColLaunchT = void (*)(const ColArgsT<T>&, int64_t grid_cap, hipStream_t);
 using RowLaunch    = RowLaunchT<float>;
 using ColLaunch    = ColLaunchT<float>;
 using XcLaunch     = void (*)(const XcArgs&, hipStream_t);
+using XcBlockLaunch = void (*)(const XcBlockArgs&, hipStream_t);
 using DifLaunch    = void (*)(const RowArgs&, int64_t batch, hipStream_t);
 using AcrossLaunch   = void (*)(const AcrossArgs&, int64_t, hipStream_t);
 using AcrossLaunch64 = void (*)(const AcrossArgsT<double>&, int64_t, hipStream_t);
@@ -94,6 +96,24 @@ void launch_xc(const XcArgs& a, hipStream_t st) {
         else
             hipLaunchKernelGGL((k_fxcorr<LA, G, false, PREC>), dim3((unsigned)nwg), dim3(NT), 0, st, s);
     }
+}
+
+// Block path of the correlation (2^15 .. 2^24): the split N1 * N2 and its three kernels.
+struct XcBlockSet {
+    int           lg, n1, n2;
+    XcBlockLaunch col_in, rows, col_out;
+};
+template<int LA, int C, int TW, bool OUT>
+void launch_xc_col(const XcBlockArgs& a, hipStream_t st) {
+    constexpr int NT  = C * Plan<LA>::TA;
+    const int64_t nwg = std::min<int64_t>(a.nb << (a.n1_lg - ilog2c(C)), 8192);
+    hipLaunchKernelGGL((k_xc_col<LA, C, TW, OUT>), dim3((unsigned)grid8(nwg)), dim3(NT), 0, st, a);
+}
+template<int LA, int TW>
+void launch_xc_rows(const XcBlockArgs& a, hipStream_t st) {
+    constexpr int G  = xc_rows<LA>();
+    constexpr int NT = G * xc_threads<LA>();
+    hipLaunchKernelGGL((k_xc_rows<LA, G, TW>), dim3((unsigned)grid8((a.nb << (a.lg - a.n1_lg)) / G)), dim3(NT), 0, st, a);
 }
 
 // Single-pass variants: 0 natural in/out; 1, 2 permuted store (forward, bit_reversed /
@@ -193,6 +213,7 @@ const std::array<std::array<RowLaunch, kMaxSinglePass - 3>, 2>& single_mfma_tab(
 const MfmaSets&                                                 single_mfma_perm_tab();
 const std::array<XcLaunch, kMaxSinglePass>& xc_tab();                         // index LA-1
 const std::array<std::array<XcLaunch, kMaxSinglePass - 3>, 2>& xc_mfma_tab(); // [prec - 1][LA - 4]
+const std::array<XcBlockSet, kMaxLog2 - kMaxSinglePass>& xc_block_tab();      // index LG-15
 const std::array<std::array<RowLaunchT<double>, 5>, kMaxSinglePass64>& single64_tab(); // index LA-1
 // four-step shapes: the defaults (first match per size), then the alternatives of the tuning
 // sweeps

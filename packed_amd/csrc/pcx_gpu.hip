@@ -969,9 +969,12 @@ struct pcx_fxcorr_s {
     int64_t    n = 0, m = 0;
     int        lg        = 0;
     int        precision = PCX_PREC_FP32;
-    float2*    tw        = nullptr; // W_N of the fused kernel (N <= 16384)
-    float*     kspec     = nullptr; // FFT(g)/N (fused kernel) or FFT(g) (block path), split re[N] im[N]
-    pcx_plan_t plan      = nullptr; // block path (N > 16384): the batched four-step FFT of size N
+    float2*    tw        = nullptr; // W_N of the fused kernel (N <= 16384), or W_N1 of the block path
+    float*     kspec     = nullptr; // FFT(g)/N, split re[N] im[N]: natural order, or the block path's rows
+    // block path (N > 16384): its kernels, W_N2 and the pass table W_N = lo[e mod 2^ls] * hi[e >> ls]
+    const XcBlockSet* blk = nullptr;
+    float2*    tw_col = nullptr, *twl = nullptr, *twh = nullptr;
+    int        tw_ls  = 0;
     // the unit's own buffers: the in-place overlap of every block (fused kernel) or the blocks in
     // flight (block path); calls on another stream than the last user wait for that use (ev)
     float*      own      = nullptr;
@@ -1022,6 +1025,14 @@ int xc_own_done(pcx_fxcorr_t x, hipStream_t st) {
     return PCX_SUCCESS;
 }
 
+// The block path's arguments that do not depend on the call.
+XcBlockArgs xc_block_args(pcx_fxcorr_t x) {
+    XcBlockArgs a{};
+    a.ksp = x->kspec, a.tw_row = x->tw, a.tw_col = x->tw_col, a.twl = x->twl, a.twh = x->twh;
+    a.lg = x->lg, a.n1_lg = x->blk->n1, a.tw_ls = x->tw_ls;
+    return a;
+}
+
 int64_t grid_of(int64_t work) { return std::max<int64_t>(1, std::min<int64_t>((work + 255) / 256, (int64_t)1 << 20)); }
 
 } // namespace
@@ -1048,39 +1059,53 @@ extern "C" int pcx_fxcorr_create(const float* g, int64_t g_pack, int64_t g_size,
     HIPCHK(setup_stream(&setup));
     auto* x = new pcx_fxcorr_s;
     x->n = fft_size, x->m = g_size, x->lg = lg;
+    x->blk        = lg > kMaxSinglePass ? &xc_block_tab()[lg - kMaxSinglePass - 1] : nullptr;
     hipError_t he = hipMalloc(&x->kspec, sizeof(float) * 2 * fft_size);
     if (he == hipSuccess)
         he = hipEventCreateWithFlags(&x->ev, hipEventDisableTiming);
-    if (he == hipSuccess && lg <= kMaxSinglePass) {
-        he = hipMalloc(&x->tw, sizeof(float2) * fft_size);
+    auto table = [&](float2** t, int64_t m, int64_t stride, int64_t count) {
         if (he == hipSuccess)
-            he = gen_twiddles(x->tw, fft_size, 1, fft_size, setup);
+            he = hipMalloc(t, sizeof(float2) * count);
         if (he == hipSuccess)
-            he = hipStreamSynchronize(setup);
+            he = gen_twiddles(*t, m, stride, count, setup);
+    };
+    const int64_t n1 = x->blk ? (int64_t)1 << x->blk->n1 : fft_size, n2 = fft_size / n1;
+    table(&x->tw, n1, 1, n1);
+    if (x->blk) {
+        x->tw_ls         = (lg + 1) / 2;
+        const int64_t nl = (int64_t)1 << x->tw_ls;
+        table(&x->tw_col, n2, 1, n2);
+        table(&x->twl, fft_size, 1, nl);
+        table(&x->twh, fft_size, nl, fft_size / nl);
+        // the two passes of FFT(g) below go through the unit's own buffer
+        if (he == hipSuccess)
+            he = hipMalloc(&x->own, sizeof(float) * 2 * fft_size);
+        x->own_cap = 2 * fft_size;
     }
+    if (he == hipSuccess)
+        he = hipStreamSynchronize(setup);
     if (he != hipSuccess) {
         pcx_fxcorr_destroy(x);
         return fail(PCX_ERR_HIP, std::string("fxcorr setup: ") + hipGetErrorString(he));
     }
-    if (lg <= kMaxSinglePass) {
-        // kernel spectrum: FFT of g zero-extended to N, scaled by 1/N (fxcorr.hpp:67-68)
-        RowArgs a{};
-        a.src = g, a.dst = x->kspec, a.src_dist = 0, a.dst_dist = 0, a.src_size = g_size, a.nrows = 1;
-        a.src_lp = ilog2(g_pack), a.dst_lp = lg, a.rows_lg = 0;
-        a.order = 0, a.conj_in = 0, a.conj_out = 0, a.scale = (float)(1.0 / (double)fft_size);
-        a.twA = x->tw;
-        single_tab()[lg - 1][0](a, 1, 0, st);
-        he = hipGetLastError();
+    // kernel spectrum: FFT of g zero-extended to N, scaled by 1/N (fxcorr.hpp:67-68); in the block
+    // path its column pass and then its rows, each stored where it stands
+    RowArgs a{};
+    a.dst = x->kspec, a.nrows = n2, a.dst_lp = lg, a.rows_lg = 0;
+    a.order = 0, a.conj_in = 0, a.conj_out = 0, a.scale = (float)(1.0 / (double)fft_size);
+    a.twA = x->tw;
+    if (x->blk) {
+        XcBlockArgs b = xc_block_args(x);
+        b.src = g, b.src_lp = ilog2(g_pack), b.len = g_size, b.step = fft_size, b.nblocks = 1, b.nb = 1, b.buf = x->own;
+        x->blk->col_in(b, st);
+        he    = hipGetLastError();
+        a.src = x->own, a.src_lp = lg, a.src_dist = n1, a.dst_dist = n1, a.src_size = n1;
     } else {
-        // block path: FFT(g) through the four-step plan; the 1/N is applied with the product
-        if (int e = pcx_plan_create(fft_size, 2048, PCX_ORDER_NORMAL, &x->plan)) {
-            pcx_fxcorr_destroy(x);
-            return e;
-        }
-        if (int e = run_batch(x->plan, 0, 0, x->kspec, fft_size, 0, g, g_pack, 0, g_size, 1, st)) {
-            pcx_fxcorr_destroy(x);
-            return e;
-        }
+        a.src = g, a.src_lp = ilog2(g_pack), a.src_size = g_size;
+    }
+    if (he == hipSuccess) {
+        single_tab()[ilog2(n1) - 1][0](a, n2, 0, st);
+        he = hipGetLastError();
     }
     if (he == hipSuccess)
         he = hipStreamSynchronize(st);
@@ -1099,10 +1124,12 @@ extern "C" int pcx_fxcorr_destroy(pcx_fxcorr_t x) {
         (void)hipEventSynchronize(x->ev);
     (void)hipFree(x->tw);
     (void)hipFree(x->kspec);
+    (void)hipFree(x->tw_col);
+    (void)hipFree(x->twl);
+    (void)hipFree(x->twh);
     (void)hipFree(x->own);
     if (x->ev)
         (void)hipEventDestroy(x->ev);
-    pcx_plan_destroy(x->plan);
     delete x;
     return PCX_SUCCESS;
 }
@@ -1166,9 +1193,10 @@ int fxcorr_run(pcx_fxcorr_t x, float* dst, int64_t dst_pack, int64_t dst_dist, c
     std::lock_guard<std::mutex> lock(x->mu);
 
     if (x->lg > kMaxSinglePass) {
-        // ---- block path: gather nb blocks, forward FFT, times conj(FFT(g)) / N, unnormalised
-        // inverse, keep `step` outputs per block.  Blocks run in increasing order, and a block's
-        // outputs lie below every later block's samples, so in place needs no saved overlap.
+        // ---- block path: column pass from the signal, rows with the product, column pass to the
+        // destination (fxcorr_kernels.hpp), nb blocks at a time.  Blocks run in increasing order,
+        // and a block's outputs lie below every later block's samples, so in place needs no saved
+        // overlap.
         float*  buf = nullptr;
         int64_t nb  = 0;
         if (ws) {
@@ -1180,22 +1208,17 @@ int fxcorr_run(pcx_fxcorr_t x, float* dst, int64_t dst_pack, int64_t dst_dist, c
                 return e;
             buf = x->own;
         }
-        XcBlockArgs a{};
-        a.src = src, a.dst = dst, a.buf = buf, a.kre = x->kspec, a.kim = x->kspec + n;
+        XcBlockArgs a = xc_block_args(x);
+        a.src = src, a.dst = dst, a.buf = buf;
         a.len = len, a.step = step, a.nblocks = nblocks, a.src_dist = src_dist, a.dst_dist = dst_dist;
-        a.src_lp = ilog2(src_pack), a.dst_lp = ilog2(dst_pack), a.lg = x->lg;
-        a.scale = (float)(1.0 / (double)n);
+        a.src_lp = ilog2(src_pack), a.dst_lp = ilog2(dst_pack);
         for (a.bg0 = 0; a.bg0 < total; a.bg0 += nb) {
             a.nb = std::min(nb, total - a.bg0);
-            hipLaunchKernelGGL(k_xc_gather, dim3((unsigned)grid_of(a.nb * n)), dim3(256), 0, st, a);
+            x->blk->col_in(a, st);
             HIPCHK(hipGetLastError());
-            if (int e = run_batch(x->plan, 0, 0, buf, n, 2 * n, (const float*)buf, n, 2 * n, n, a.nb, st))
-                return e;
-            hipLaunchKernelGGL(k_xc_mul, dim3((unsigned)grid_of(a.nb * n)), dim3(256), 0, st, a);
+            x->blk->rows(a, st);
             HIPCHK(hipGetLastError());
-            if (int e = run_batch(x->plan, 1, 0, buf, n, 2 * n, (const float*)buf, n, 2 * n, n, a.nb, st))
-                return e;
-            hipLaunchKernelGGL(k_xc_scatter, dim3((unsigned)grid_of(a.nb * step)), dim3(256), 0, st, a);
+            x->blk->col_out(a, st);
             HIPCHK(hipGetLastError());
         }
         return ws ? PCX_SUCCESS : xc_own_done(x, st);

@@ -188,6 +188,29 @@ def test_block_path_above_16384(orc, pa, L, M, N, inplace):
     assert orc.rel_l2(got, orc.xcorr_naive(f, g)) < 4e-6
 
 
+@pytest.mark.parametrize("lg,sp,dp", [(15, 8, 8), (15, 1, 1 << 15), (16, 64, 8), (17, 8, 1 << 20), (18, 1, 8),
+                                      (19, 8, 8), (20, 1024, 16), (21, 8, 8), (22, 8, 8), (23, 8, 8), (24, 8, 8)])
+def test_block_path_every_size(orc, pa, lg, sp, dp):
+    """Every block size above 16384, out of place, two blocks of which the second holds 77 samples;
+    packs of both vectors on either side of the column tiles' width, and destination packs that the
+    block offset is no multiple of.  Reference: the FP64 correlation through numpy's FFT."""
+    import torch
+
+    n = 1 << lg
+    m = n // 3 + 1
+    length = (n - m + 1) // sp * sp + 77
+    f = orc.gen_normal(0x5EED0081, length, np.sqrt(0.5)).astype(np.complex64)
+    g = np.exp(1j * np.pi * np.real(orc.gen_uniform(0x5EED0082, m))).astype(np.complex64)
+    out = pa.vector(length, dp)
+    pa.fxcorr_unit(pa.vector.from_complex(g, sp), n)(pa.vector.from_complex(f, sp), out)
+    torch.cuda.synchronize()
+    s = 1 << (length + m).bit_length()
+    want = np.fft.ifft(np.fft.fft(f.astype(np.complex128), s) * np.conj(np.fft.fft(g.astype(np.complex128), s)))
+    got = out.to_complex()
+    assert orc.rel_l2(got, want[:length]) < 4e-6
+    assert orc.rel_l2(got[-77:], want[length - 77:length]) < 4e-6 * np.sqrt(length)
+
+
 @pytest.mark.parametrize("L,M,N,C", [(20000, 300, 1024, 3), (3000, 57, 128, 4), (150000, 20000, 1 << 15, 2),
                                      (100000, 10, 64, 2), (30000, 150, 256, 3)])
 @pytest.mark.parametrize("inplace", [True, False])
