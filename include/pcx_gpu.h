@@ -75,14 +75,15 @@ int     pcx_plan_precision(pcx_plan_t plan);
  * blocking; these pick the GPU's.  None changes results.
  * pcx_plan_set_shape: one of the instantiated N1 x N2 splits and tiles: column length
  *   2^n2_log2, `cols` columns per column tile, `rows` rows per row workgroup (0 = any; the first
- *   listed match wins, the default first).  Rebuilds the split's twiddle tables after a
+ *   listed match wins, the default first; all 0: the default, and smaller tiles of its split for
+ *   calls of few points, which a plan starts with).  Rebuilds the split's twiddle tables after a
  *   device-wide synchronisation (every enqueued use of the old tables ends first).  Split-
  *   precision plans keep the default shape.
  * pcx_plan_shape: the current split and tiles (0s for a single-pass plan).
  * pcx_plan_set_grid: workgroup caps of the column and row passes (0 = one per tile; the kernels
- *   loop over the rest).  pcx_plan_set_chunk: bytes of the intermediate of one chunk of a batch
- *   (0 = the default 2 GiB).  pcx_plan_set_one_pass: 2^15 runs as one decimation-in-frequency
- *   pass (default on) or as the four-step.  pcx_plan_set_three_pass: natural-order transforms
+ *   loop over the rest; a plan starts with 2048 for tiles that fill a CU and none for smaller).  pcx_plan_set_chunk: bytes of the intermediate of one chunk of a batch
+ *   (0 = the default 2 GiB).  pcx_plan_set_one_pass: calls of 48 or more 2^15-point FP32
+ *   transforms run in one pass (default on) or as the four-step.  pcx_plan_set_three_pass: natural-order transforms
  *   of 2^21 .. 2^24 points (FP64: 2^21 .. 2^23) run in three passes over the intermediate
  *   (default on) or as the four-step (the permuted orders always take the four-step). */
 int pcx_plan_set_shape(pcx_plan_t plan, int n2_log2, int cols, int rows);

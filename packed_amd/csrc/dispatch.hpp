@@ -24,6 +24,10 @@ constexpr int kMaxLog2         = 24; // four-step limit: N2 <= 2048 columns, N1 
 constexpr int kMaxSinglePass64 = 13; // FP64: N <= 8192 in one pass
 constexpr int kMaxLog2_64      = 23; // FP64 four-step limit
 constexpr int kDifLog2         = 15; // one-pass decimation-in-frequency size
+// Sizes beyond the single pass whose transform still fits a CU's LDS as one array (128 KiB): calls
+// of enough transforms run them in one pass, one workgroup per transform (one_pass_tab).
+constexpr int kOnePassLog2     = 15;
+constexpr int kOnePassLog2_64  = 14;
 constexpr int kMaxAcross       = 13; // transforms across at most 8192 vectors (float)
 constexpr int kMaxAcross64     = 11; // and 2048 vectors (double)
 
@@ -51,14 +55,14 @@ inline int64_t fit_grid(int64_t nwg, int64_t threads) {
 inline int64_t pidx64(int64_t i, int lp) { return i + ((i >> lp) << lp); }
 
 template<int LA, int G, int LD, int ST, int TW, bool UNI = (Plan<LA>::TA >= 64), int ORD = 0, int PREC = PREC_FP32,
-         class T = float>
+         class T = float, int PX = 0>
 void launch_row(const RowArgsT<T>& a, int64_t nrows, int64_t grid_cap, hipStream_t st) {
-    int64_t nwg = (nrows + G - 1) / G;
+    constexpr int NT  = G * Plan<LA, false, T, PX>::TA;
+    int64_t       nwg = (nrows + G - 1) / G;
     if (grid_cap > 0 && nwg > grid_cap)
         nwg = grid_cap;
-    nwg = fit_grid(grid8(nwg), G * Plan<LA, false, T>::TA);
-    hipLaunchKernelGGL((k_row<LA, G, LD, ST, TW, UNI, ORD, PREC, T>), dim3((unsigned)nwg),
-                       dim3(G * Plan<LA, false, T>::TA), 0, st, a);
+    nwg = fit_grid(grid8(nwg), NT);
+    hipLaunchKernelGGL((k_row<LA, G, LD, ST, TW, UNI, ORD, PREC, T, PX>), dim3((unsigned)nwg), dim3(NT), 0, st, a);
 }
 template<int LA, int C, int TW, int PREC = PREC_FP32, class T = float, int PX = 0>
 void launch_col(const ColArgsT<T>& a, int64_t grid_cap, hipStream_t st) {
@@ -182,8 +186,25 @@ struct FourStepT {
     int                          lg, n1, n2, g, c;
     std::array<RowLaunchT<T>, 6> rows;
     std::array<ColLaunchT<T>, 2> cols;
+    // default grid cap: workgroups that fill a CU by themselves loop over their tiles (2048);
+    // several smaller ones per CU run one tile each (0: no cap), the next workgroup's loads
+    // overlapping the others' stores (2^16 x 1024, 4096-point tiles: 429 us against 539 capped)
+    int64_t grid = 0;
 };
 using FourStep = FourStepT<float>;
+constexpr int64_t kWideGrid = 2048;
+// Shapes for calls of at most 2^max_lg points over all their transforms, with the same split as
+// the default shape of their size and smaller tiles; the first match per size and split.
+template<class T>
+struct SmallShapeT {
+    int          max_lg;
+    FourStepT<T> f;
+};
+template<class T>
+struct SmallList {
+    const SmallShapeT<T>* data;
+    int                   count;
+};
 
 // Split-precision matrix-core variants of the default shapes for 2^15 .. 2^20 (natural order):
 // index [precision - 1], rows {forward, inverse}, cols {inverse, forward}
@@ -215,12 +236,16 @@ const std::array<XcLaunch, kMaxSinglePass>& xc_tab();                         //
 const std::array<std::array<XcLaunch, kMaxSinglePass - 3>, 2>& xc_mfma_tab(); // [prec - 1][LA - 4]
 const std::array<XcBlockSet, kMaxLog2 - kMaxSinglePass>& xc_block_tab();      // index LG-15
 const std::array<std::array<RowLaunchT<double>, 5>, kMaxSinglePass64>& single64_tab(); // index LA-1
+const RowSet&                            one_pass_tab();   // 2^15, variants as single_tab's
+const std::array<RowLaunchT<double>, 5>& one_pass64_tab(); // FP64 2^14
 // four-step shapes: the defaults (first match per size), then the alternatives of the tuning
 // sweeps
 ShapeList<float>  shapes_default();
 ShapeList<float>  shapes_alt();
 ShapeList<double> shapes64_default();
 ShapeList<double> shapes64_alt();
+SmallList<float>  shapes_small();   // k_shapes_small.hip
+SmallList<double> shapes64_small();
 const std::array<FourStepMfma, 6>& shapes_mfma();
 // permuted-order row kernels of those shapes (k_mfma_p4.hip): [shape][precision - 1]
 // {forward bit_reversed, forward unordered, inverse bit_reversed, inverse unordered}

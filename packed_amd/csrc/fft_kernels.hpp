@@ -768,9 +768,9 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
 }
 
 // LDS elements (of T) of a row workgroup
-template<int LA, int G, int TW, class T = float>
+template<int LA, int G, int TW, class T = float, int PX = 0>
 constexpr int row_lds_floats() {
-    return RowShape<LA, G, T>::DATA + TwTable<LA, T>::FLOATS + 2 * TW;
+    return RowShape<LA, G, T, PX>::DATA + TwTable<LA, T>::FLOATS + 2 * TW;
 }
 
 // Grid-stride over row groups: gridDim.x may be smaller than the number of groups.
@@ -778,19 +778,19 @@ constexpr int row_lds_floats() {
 // but at least two, so the register budget (256) never pushes accumulators into AGPRs.
 constexpr int mfma_waves(int w, int prec) { return prec == PREC_FP32 ? w : (w > 4 ? w / 2 : 2); }
 
-template<int LA, int G, int LD, int ST, int TW, bool UNI, int ORD, int PREC = PREC_FP32, class T = float>
-__global__ __launch_bounds__((G * Plan<LA, false, T>::TA),
-                             mfma_waves(waves_per_simd(G * Plan<LA, false, T>::TA,
-                                                       (int)sizeof(T) * row_lds_floats<LA, G, TW, T>()),
+template<int LA, int G, int LD, int ST, int TW, bool UNI, int ORD, int PREC = PREC_FP32, class T = float, int PX = 0>
+__global__ __launch_bounds__((G * Plan<LA, false, T, PX>::TA),
+                             mfma_waves(waves_per_simd(G * Plan<LA, false, T, PX>::TA,
+                                                       (int)sizeof(T) * row_lds_floats<LA, G, TW, T, PX>()),
                                         PREC))
 void k_row(RowArgsT<T> p) {
-    constexpr int NT = G * Plan<LA, false, T>::TA;
-    __shared__ T  lds[row_lds_floats<LA, G, TW, T>()];
-    using LC           = LdsCarve<T, RowShape<LA, G, T>::DATA, TwTable<LA, T>::FLOATS, 2 * TW>;
+    constexpr int NT = G * Plan<LA, false, T, PX>::TA;
+    __shared__ T  lds[row_lds_floats<LA, G, TW, T, PX>()];
+    using LC           = LdsCarve<T, RowShape<LA, G, T, PX>::DATA, TwTable<LA, T>::FLOATS, 2 * TW>;
     T*            ltw  = lds + LC::TOFF;
     T*            lptw = ltw + TwTable<LA, T>::FLOATS;
     T*            lre  = lds + LC::DOFF;
-    T*            lim  = RowShape<LA, G, T>::im(lre);
+    T*            lim  = RowShape<LA, G, T, PX>::im(lre);
     TwTable<LA, T>::fill(ltw, p.twA, threadIdx.x, NT);
     if constexpr (TW > 0)
         PassTw<TW, T>::fill(lptw, p.twl, p.twh, p.tw_ls, p.tw_lg, threadIdx.x, NT);
@@ -803,7 +803,7 @@ void k_row(RowArgsT<T> p) {
         const int64_t wg = xcd_item(base);
         if (wg >= nwg)
             break; // uniform over the workgroup; later rounds have no items for it either
-        row_group<LA, G, LD, ST, TW, UNI, ORD, PREC, T>(p, wg, lre, lim, ltw, lptw, &mf);
+        row_group<LA, G, LD, ST, TW, UNI, ORD, PREC, T, PX>(p, wg, lre, lim, ltw, lptw, &mf);
         __syncthreads(); // LDS is reused by the next group
     }
 }

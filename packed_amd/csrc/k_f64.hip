@@ -7,14 +7,14 @@ namespace {
 
 // ---- fft_unit<double, Order>: natural and bit_reversed orders (the reference has no FP64
 // unordered kernel: avx2_fft.hpp:114-217 is written for float only)
-template<int LA>
+template<int LA, int PX = 0>
 constexpr std::array<RowLaunchT<double>, 5> single_set64() {
     using D            = double;
-    constexpr int  G   = default_rows<LA, D>();
-    constexpr bool UNI = Plan<LA, false, D>::TA >= 64;
-    return {&launch_row<LA, G, LD_CONTIG, ST_CONTIG, 0, UNI, 0, PREC_FP32, D>,
-            &launch_row<LA, G, LD_CONTIG, ST_PERM, 0, UNI, ORD_BITREV, PREC_FP32, D>, nullptr,
-            &launch_row<LA, G, LD_PERM, ST_CONTIG, 0, UNI, ORD_BITREV, PREC_FP32, D>, nullptr};
+    constexpr int  G   = Plan<LA, false, D, PX>::TA >= 256 ? 1 : 256 / Plan<LA, false, D, PX>::TA;
+    constexpr bool UNI = Plan<LA, false, D, PX>::TA >= 64;
+    return {&launch_row<LA, G, LD_CONTIG, ST_CONTIG, 0, UNI, 0, PREC_FP32, D, PX>,
+            &launch_row<LA, G, LD_CONTIG, ST_PERM, 0, UNI, ORD_BITREV, PREC_FP32, D, PX>, nullptr,
+            &launch_row<LA, G, LD_PERM, ST_CONTIG, 0, UNI, ORD_BITREV, PREC_FP32, D, PX>, nullptr};
 }
 template<int... L>
 constexpr auto single_table64(std::integer_sequence<int, L...>) {
@@ -29,8 +29,9 @@ constexpr auto single_table64(std::integer_sequence<int, L...>) {
 // against 3.23 ms for C = 8, G = 2.
 constexpr FourStepT<double> kDefault64[] = {
     shape64<14, 7, 7, 32, 64>(), shape64<15, 8, 7, 32, 64>(), shape64<16, 8, 8, 32, 32>(),
-    shape64<17, 8, 9, 32, 16>(),  // 1.84 ms
-    shape64<18, 10, 8, 8, 32>(),  // 1.89
+    // 4096-point tiles, up to two workgroups per CU and one tile each: 2^26 points 881 / 900 and
+    // 972 / 920 us forward / inverse against 944 / 942 (8, 9, 32, 16) and 961 / 985 (10, 8, 8, 32)
+    shape64<17, 9, 8, 8, 16>(), shape64<18, 9, 9, 8, 8>(),
     shape64<19, 10, 9, 8, 16>(),  // 2.41
     shape64<20, 10, 10, 8, 8>(),  // 2.43
     shape64<21, 11, 10, 4, 8>(),  // 3.11
@@ -40,6 +41,9 @@ constexpr FourStepT<double> kDefault64[] = {
 
 const std::array<std::array<RowLaunchT<double>, 5>, kMaxSinglePass64> kSingle64 =
     single_table64(std::make_integer_sequence<int, kMaxSinglePass64>{});
+
+// 2^14 doubles in one pass: 16 points per thread, 1024 threads, 132 KiB of LDS (one array).
+const std::array<RowLaunchT<double>, 5> kOnePass64 = single_set64<kOnePassLog2_64, 16>();
 
 // Three-pass natural-order transforms of 2^21 .. 2^23 doubles: tiles of 8192 points (128 KiB),
 // first-pass columns of 2^7 / 2^8 (64 / 32 per tile, 512- / 256-byte segments), 64 second-pass
@@ -59,6 +63,7 @@ constexpr ThreePassT<double> kThree64[] = {three_pass64<21, 7, 7>(), three_pass6
 } // namespace
 
 const std::array<std::array<RowLaunchT<double>, 5>, kMaxSinglePass64>& single64_tab() { return kSingle64; }
+const std::array<RowLaunchT<double>, 5>& one_pass64_tab() { return kOnePass64; }
 ShapeList<double> shapes64_default() { return {kDefault64, (int)(sizeof(kDefault64) / sizeof(kDefault64[0]))}; }
 ThreeList<double> three_pass64_tab() { return {kThree64, (int)(sizeof(kThree64) / sizeof(kThree64[0]))}; }
 

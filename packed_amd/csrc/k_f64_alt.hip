@@ -5,10 +5,10 @@
 namespace pcxd {
 namespace {
 constexpr FourStepT<double> kAlt64[] = {
-    shape64<17, 9, 8, 8, 16>(),   // 2.08
+    shape64<17, 8, 9, 32, 16>(),
     shape64<17, 9, 8, 16, 16>(),  // 1.90 (inverse 2.05)
     shape64<18, 10, 8, 4, 16>(),  // 2.71
-    shape64<18, 9, 9, 8, 8>(),    // 2.22
+    shape64<18, 10, 8, 8, 32>(),
     shape64<18, 8, 10, 16, 4>(),  // 2.15
     shape64<19, 10, 9, 4, 8>(),   // 3.25
     shape64<19, 9, 10, 8, 4>(),   // 2.81

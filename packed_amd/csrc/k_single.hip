@@ -5,13 +5,28 @@
 namespace pcxd {
 namespace {
 
+// Plan options of the largest single passes: 16 points per thread and one exchange array (35 KiB,
+// four workgroups of 512 threads per CU, at 2^13; 66 KiB, two of 1024 threads, at 2^14).  They
+// are bound by the exchanges' latency for few transforms and by HBM for many, and more waves per CU
+// help both.  us for 1 / 1024 / 16384 transforms (pack 8, forward), 32 points per thread and two
+// arrays at 2^13, 64 points at 2^14, against these: 2^13 8.7 / 31.9 / 414 -> 7.8 / 27.5 / 386,
+// 2^14 17.7 / 60.7 / 793 -> 12.5 / 52.8 / 729.
 template<int LA>
+constexpr int single_px() {
+    return LA == 14 ? 16 : (LA == 13 ? 16 | kHalfExchange : 0);
+}
+// 2^15 points in one pass: 32 points per thread, 1024 threads, 132 KiB of LDS (one array).
+constexpr int kOnePassPx = 32 | kTwChain;
+
+template<int LA, int PX = single_px<LA>()>
 constexpr RowSet single_set() {
-    constexpr int  G   = default_rows<LA>();
-    constexpr bool UNI = Plan<LA>::TA >= 64;
-    return {&launch_row<LA, G, LD_CONTIG, ST_CONTIG, 0, UNI, 0>, &launch_row<LA, G, LD_CONTIG, ST_PERM, 0, UNI, ORD_BITREV>,
-            &launch_row<LA, G, LD_CONTIG, ST_PERM, 0, UNI, ORD_UNORD>, &launch_row<LA, G, LD_PERM, ST_CONTIG, 0, UNI, ORD_BITREV>,
-            &launch_row<LA, G, LD_PERM, ST_CONTIG, 0, UNI, ORD_UNORD>};
+    constexpr int  G   = Plan<LA, false, float, PX>::TA >= 256 ? 1 : 256 / Plan<LA, false, float, PX>::TA;
+    constexpr bool UNI = Plan<LA, false, float, PX>::TA >= 64;
+    return {&launch_row<LA, G, LD_CONTIG, ST_CONTIG, 0, UNI, 0, PREC_FP32, float, PX>,
+            &launch_row<LA, G, LD_CONTIG, ST_PERM, 0, UNI, ORD_BITREV, PREC_FP32, float, PX>,
+            &launch_row<LA, G, LD_CONTIG, ST_PERM, 0, UNI, ORD_UNORD, PREC_FP32, float, PX>,
+            &launch_row<LA, G, LD_PERM, ST_CONTIG, 0, UNI, ORD_BITREV, PREC_FP32, float, PX>,
+            &launch_row<LA, G, LD_PERM, ST_CONTIG, 0, UNI, ORD_UNORD, PREC_FP32, float, PX>};
 }
 template<int... L>
 constexpr auto single_table(std::integer_sequence<int, L...>) {
@@ -56,6 +71,7 @@ constexpr auto across_table(std::integer_sequence<int, L...>) {
 }
 
 const std::array<RowSet, kMaxSinglePass> kSingle = single_table(std::make_integer_sequence<int, kMaxSinglePass>{});
+const RowSet kOnePass = single_set<kOnePassLog2, kOnePassPx>();
 const std::array<DifLaunch, 3> kDif = {&launch_dif<14, 1, ORD_NORMAL>, &launch_dif<13, 2, ORD_BITREV>,
                                        &launch_dif<13, 2, ORD_UNORD>};
 const std::array<AcrossLaunch, kMaxAcross> kAcross =
@@ -66,6 +82,7 @@ const std::array<AcrossLaunch64, kMaxAcross64> kAcross64 =
 } // namespace
 
 const std::array<RowSet, kMaxSinglePass>& single_tab() { return kSingle; }
+const RowSet&                               one_pass_tab() { return kOnePass; }
 const std::array<DifLaunch, 3>&            dif_tab() { return kDif; }
 const std::array<AcrossLaunch, kMaxAcross>& across_tab() { return kAcross; }
 const std::array<AcrossLaunch64, kMaxAcross64>& across64_tab() { return kAcross64; }

@@ -137,6 +137,16 @@ const FourStepT<double>* find_shape64(int lg, int n2, int g, int c) {
         return f;
     return find_in(shapes64_alt(), lg, n2, g, c);
 }
+// The small-tile shape for a call of `points` points with the plan's split, or null.
+template<class T>
+const FourStepT<T>* find_small(const SmallList<T>& l, const FourStepT<T>* sh, int64_t points) {
+    for (int i = 0; i < l.count; ++i) {
+        const SmallShapeT<T>& e = l.data[i];
+        if (e.f.lg == sh->lg && e.f.n1 == sh->n1 && points <= ((int64_t)1 << e.max_lg))
+            return &e.f;
+    }
+    return nullptr;
+}
 // The same for FP64: bit_reversed 2^21 .. 2^23 take rows of 2^13 points, one per workgroup, and
 // the widest column tiles (per 2 GiB, forward / inverse: 2.02 / 1.92, 2.06 / 2.14, 2.53 / 2.61 ms
 // against 2.41 / 2.47, 2.53 / 2.64, 4.23 / 4.44 with the first listed shapes).
@@ -188,11 +198,16 @@ struct pcx_plan_s {
     int64_t chunk        = 0; // transforms per four-step chunk
     const FourStep* shape = nullptr; // four-step kernels and tile sizes
     int     precision    = PCX_PREC_FP32;
-    int64_t grid_col     = 2048; // grid caps of the two passes (persistent loop; 0: one workgroup per tile)
-    int64_t grid_row     = 2048;
+    // grid caps of the two passes (persistent loop; 0: one workgroup per tile; -1: the shape's own)
+    int64_t grid_col     = -1;
+    int64_t grid_row     = -1;
+    bool    auto_shape   = true; // no shape was chosen by the caller: calls of few points take small tiles
     int     nt_flags     = 0; // bit 0/1: streaming load/store of src/dst, bit 2/3: of the intermediate
     float2* tw_dif       = nullptr; // W_M for the one-pass k_dif kernel
-    bool    use_dif      = false;   // out-of-place transforms of 2^15 run as one k_dif pass
+    // one-pass forms of 2^15 (FP64: 2^14) points (pcx_plan_set_one_pass): one workgroup per
+    // transform (W_N in tw_one), or k_dif
+    bool    use_one      = false;
+    void*   tw_one       = nullptr;
     // three-pass natural-order transforms of 2^21 .. 2^24 (FP64: 2^21 .. 2^23): stage tables
     // W_N2, W_Nb, W_Na and the two-level W_N1 pass table (lo, hi), in the plan's precision
     bool    use_three    = false;
@@ -308,13 +323,17 @@ extern "C" int pcx_plan_create(int64_t fft_size, int64_t sub_size, int order, pc
         he       = fourstep_tables(p, st);
         // transforms per four-step chunk: the intermediate holds one chunk
         p->chunk = std::max<int64_t>(1, kChunkBytes / (fft_size * 8));
-        if (lg == kDifLog2) {
-            p->use_dif     = true;
+        if (lg == kOnePassLog2) {
+            p->use_one      = true;
             const int64_t m = (int64_t)1 << dif_core_log2(order);
             if (he == hipSuccess)
                 he = hipMalloc(&p->tw_dif, sizeof(float2) * m);
             if (he == hipSuccess)
                 he = gen_twiddles(p->tw_dif, m, 1, m, st);
+            if (he == hipSuccess)
+                he = hipMalloc(&p->tw_one, sizeof(float2) * fft_size);
+            if (he == hipSuccess)
+                he = gen_twiddles((float2*)p->tw_one, fft_size, 1, fft_size, st);
         }
         // three passes are the default: 2^21 / 2^22 / 2^23 / 2^24 in 2.74 / 2.83 / 2.93 /
         // 2.95 ms per 2 GiB forward against 3.03 / 3.67 / 4.45 / 6.00 with the four-step
@@ -345,6 +364,7 @@ extern "C" int pcx_plan_destroy(pcx_plan_t p) {
     (void)hipFree(p->twh);
     (void)hipFree(p->tmp);
     (void)hipFree(p->tw_dif);
+    (void)hipFree(p->tw_one);
     for (void* t : p->tw3)
         (void)hipFree(t);
     (void)hipFree(p->tw64_row);
@@ -410,6 +430,13 @@ extern "C" int pcx_plan_create_f64(int64_t fft_size, int64_t sub_size, int order
         if (he == hipSuccess)
             he = gen_twiddles(p->twh64, fft_size, nl, nh, st);
         p->chunk = std::max<int64_t>(1, kChunkBytes / (fft_size * 16));
+        if (lg == kOnePassLog2_64) {
+            p->use_one = true;
+            if (he == hipSuccess)
+                he = hipMalloc(&p->tw_one, sizeof(double2) * fft_size);
+            if (he == hipSuccess)
+                he = gen_twiddles((double2*)p->tw_one, fft_size, 1, fft_size, st);
+        }
         if (he == hipSuccess)
             he = three_pass_tables<double>(p, st);
         if (he == hipSuccess)
@@ -521,6 +548,14 @@ struct ExtTmp {
     int64_t bytes;
 };
 
+// Transforms from which a call of 2^15 points (FP64: 2^14) runs one workgroup per transform, and
+// from which 2^15 runs as k_dif before that; fewer transforms spread over the chip as small
+// four-step tiles.  2^15, forward, pack 8, four-step / k_dif / one pass, us: 1 transform 14.6 / 20.2 / 22.4,
+// 32 16.4 / 21.6 / -, 64 22.7 / 23.7 / 25.5, 256 51 / 41.9 / 36.9, 1024 248 / 188 / 159, 4096 (2^27
+// points) - / 710 / 546; bit_reversed 64 23.1 / 18.8 / 29.8, 256 51 / 43.9 / 40.6, 1024
+// 264 / 199 / 181.  FP64 2^14, four-step / one pass: 64 19.1 / 23.3, 256 48 / 32.3, 4096 790 / 484.
+constexpr int64_t kOnePassBatch = 160, kDifBatch = 48, kOnePassBatch64 = 96;
+
 // src_offs / dst_offs (optional, device arrays of `batch` element offsets) replace b * dist.
 // T is the element type: float, or double for a plan made by pcx_plan_create_f64.
 template<class T>
@@ -573,28 +608,33 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
     else
         tw_row = p->tw_row, tw_col = p->tw_col, twl = p->twl, twh = p->twh;
 
-    if (!p->two_pass) {
+    // ---- one pass: one workgroup (or several, for small sizes) per group of whole transforms
+    const bool whole = p->use_one && p->precision == PCX_PREC_FP32 && batch >= (F64 ? kOnePassBatch64 : kOnePassBatch);
+    if (!p->two_pass || whole) {
         RowArgsT<T> a{};
         a.src = src, a.dst = dst, a.src_dist = src_dist, a.dst_dist = dst_dist;
         a.src_size = src_size, a.nrows = batch, a.src_lp = src_lp, a.dst_lp = dst_lp, a.rows_lg = 0;
         a.order = p->order, a.conj_in = inverse, a.conj_out = inverse, a.scale = scale;
-        a.twA = tw_row, a.twl = nullptr, a.twh = nullptr, a.tw_ls = 0;
+        a.twA = whole ? (const vec2<T>*)p->tw_one : tw_row, a.twl = nullptr, a.twh = nullptr, a.tw_ls = 0;
         a.src_offs = src_offs, a.dst_offs = dst_offs;
+        const int v = single_variant(inverse, p->order);
         if constexpr (F64)
-            single64_tab()[p->lg - 1][single_variant(inverse, p->order)](a, batch, 0, st);
+            (whole ? one_pass64_tab() : single64_tab()[p->lg - 1])[v](a, batch, 0, st);
+        else if (whole)
+            one_pass_tab()[v](a, batch, 0, st);
         else if (p->precision != PCX_PREC_FP32 && p->order == PCX_ORDER_NORMAL)
             single_mfma_tab()[p->precision - 1][p->lg - 4](a, batch, 0, st);
         else if (p->precision != PCX_PREC_FP32)
-            single_mfma_perm_tab()[p->precision - 1][p->lg - 4][single_variant(inverse, p->order)](a, batch, 0, st);
+            single_mfma_perm_tab()[p->precision - 1][p->lg - 4][v](a, batch, 0, st);
         else
-            single_tab()[p->lg - 1][single_variant(inverse, p->order)](a, batch, 0, st);
+            single_tab()[p->lg - 1][v](a, batch, 0, st);
         HIPCHK(hipGetLastError());
         return PCX_SUCCESS;
     }
 
     // ---- one pass, radix-R decimation in frequency + M-point Stockham (no intermediate)
     if constexpr (!F64)
-    if (p->use_dif && p->precision == PCX_PREC_FP32 && (const float*)dst != src &&
+    if (p->use_one && p->precision == PCX_PREC_FP32 && batch >= kDifBatch && (const float*)dst != src &&
         (!inverse || p->order == PCX_ORDER_NORMAL)) {
         RowArgs a{};
         a.src = src, a.dst = dst, a.src_dist = src_dist, a.dst_dist = dst_dist;
@@ -647,10 +687,15 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
         tmp = reinterpret_cast<T*>(p->tmp);
     }
     const FourStepT<T>* shape;
+    SmallList<T>        small;
     if constexpr (F64)
-        shape = p->shape64;
+        shape = p->shape64, small = shapes64_small();
     else
-        shape = p->shape;
+        shape = p->shape, small = shapes_small();
+    // by the whole call, not the chunk: every chunk size then runs the same kernels
+    if (p->auto_shape && p->precision == PCX_PREC_FP32)
+        if (const FourStepT<T>* f = find_small(small, shape, batch << p->lg))
+            shape = f;
     int           C    = shape->c;
     ColLaunchT<T> colf = shape->cols[inverse ? 0 : 1];
     RowLaunchT<T> rowf = shape->rows[(inverse ? 3 : 0) + p->order];
@@ -676,6 +721,9 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
     const ThreePassT<T>* tp3 = p->use_three && p->order == PCX_ORDER_NORMAL && p->precision == PCX_PREC_FP32
                                    ? three_of<T>(p->lg)
                                    : nullptr;
+    const int64_t own_grid = tp3 || p->precision != PCX_PREC_FP32 ? kWideGrid : shape->grid;
+    const int64_t grid_col = p->grid_col >= 0 ? p->grid_col : own_grid;
+    const int64_t grid_row = p->grid_row >= 0 ? p->grid_row : own_grid;
     for (int64_t b0 = 0; b0 < batch; b0 += chunk) {
         int64_t      cb = batch - b0 < chunk ? batch - b0 : chunk;
         const T*       cs  = src_offs ? src : src + b0 * src_dist;
@@ -694,21 +742,21 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
             c1.ntiles = cb * (m1 / tp3->c1), c1.n1_lg = l1, c1.conj_in = inverse, c1.conj_out = 0, c1.scale = T(1);
             c1.twA = (const V*)p->tw3[0], c1.twl = twl, c1.twh = twh, c1.tw_ls = p->tw_ls, c1.tw_lg = p->lg;
             c1.nt_load = p->nt_flags & 1, c1.nt_store = (p->nt_flags >> 2) & 1;
-            tp3->col1(c1, p->grid_col, st);
+            tp3->col1(c1, grid_col, st);
             c2.src = tmp, c2.src_dist = 2 * m1, c2.src_lp = l1, c2.src_size = m1;
             c2.dst = tmp, c2.dst_dist = 2 * m1, c2.dst_lp = l1;
             c2.ntiles = (cb << tp3->n2_lg) * (((int64_t)1 << tp3->na_lg) / tp3->c2), c2.n1_lg = tp3->na_lg;
             c2.conj_in = 0, c2.conj_out = 0, c2.scale = T(1);
             c2.twA = (const V*)p->tw3[1], c2.twl = (const V*)p->tw3[3], c2.twh = (const V*)p->tw3[4];
             c2.tw_ls = p->tw_ls1, c2.tw_lg = l1;
-            tp3->col2(c2, p->grid_col, st);
+            tp3->col2(c2, grid_col, st);
             r3.src = tmp, r3.src_dist = 2 * n, r3.src_lp = l1, r3.src_size = n;
             r3.dst = cd, r3.dst_dist = dst_dist, r3.dst_lp = dst_lp, r3.dst_offs = cdo;
             r3.rows_lg = p->lg - tp3->na_lg, r3.rsplit_lg = tp3->n2_lg, r3.nrows = cb << (p->lg - tp3->na_lg);
             r3.order = PCX_ORDER_NORMAL, r3.conj_in = 0, r3.conj_out = inverse, r3.scale = scale;
             r3.twA = (const V*)p->tw3[2];
             r3.nt_load = (p->nt_flags >> 3) & 1, r3.nt_store = (p->nt_flags >> 1) & 1;
-            tp3->row3(r3, r3.nrows, p->grid_row, st);
+            tp3->row3(r3, r3.nrows, grid_row, st);
             HIPCHK(hipGetLastError());
             continue;
         }
@@ -724,14 +772,14 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
             ca.conj_in = 0, ca.conj_out = 0, ca.scale = T(1);
             ca.twl = twl, ca.twh = twh, ca.tw_ls = p->tw_ls;
             ca.nt_load = p->nt_flags & 1, ca.nt_store = (p->nt_flags >> 2) & 1;
-            colf(ca, p->grid_col, st);
+            colf(ca, grid_col, st);
             // pass B: rows of the intermediate -> dst in the plan's order
             ra.src = tmp, ra.src_dist = 2 * n, ra.src_lp = p->lg, ra.src_size = n;
             ra.dst = cd, ra.dst_dist = dst_dist, ra.dst_lp = dst_lp, ra.dst_offs = cdo;
             ra.conj_in = 0, ra.conj_out = 0, ra.scale = T(1);
             ra.twl = nullptr, ra.twh = nullptr;
             ra.nt_load = (p->nt_flags >> 3) & 1, ra.nt_store = (p->nt_flags >> 1) & 1;
-            rowf(ra, ra.nrows, p->grid_row, st);
+            rowf(ra, ra.nrows, grid_row, st);
         } else {
             // pass 1: rows (over k1) of the spectrum -> intermediate, times W_N^(n1*k2)
             ra.src = cs, ra.src_dist = src_dist, ra.src_lp = src_lp, ra.src_size = n, ra.src_offs = cso;
@@ -739,14 +787,14 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
             ra.conj_in = 1, ra.conj_out = 0, ra.scale = T(1);
             ra.twl = twl, ra.twh = twh, ra.tw_ls = p->tw_ls;
             ra.nt_load = p->nt_flags & 1, ra.nt_store = (p->nt_flags >> 2) & 1;
-            rowf(ra, ra.nrows, p->grid_row, st);
+            rowf(ra, ra.nrows, grid_row, st);
             // pass 2: columns (over k2) of the intermediate -> dst, natural order
             ca.src = tmp, ca.src_dist = 2 * n, ca.src_lp = p->lg, ca.src_size = n;
             ca.dst = cd, ca.dst_dist = dst_dist, ca.dst_lp = dst_lp, ca.dst_offs = cdo;
             ca.conj_in = 0, ca.conj_out = 1, ca.scale = scale;
             ca.twl = nullptr, ca.twh = nullptr;
             ca.nt_load = (p->nt_flags >> 3) & 1, ca.nt_store = (p->nt_flags >> 1) & 1;
-            colf(ca, p->grid_col, st);
+            colf(ca, grid_col, st);
         }
         HIPCHK(hipGetLastError());
     }
@@ -781,12 +829,17 @@ extern "C" int pcx_plan_set_shape(pcx_plan_t p, int n2_log2, int cols, int rows)
         const FourStepT<double>* sh = find_shape64(p->lg, n2_log2, rows, cols);
         if (!sh)
             return fail(PCX_ERR_UNSUPPORTED, "no double four-step shape of fft_size " + s(p->n) + " matches");
-        return plan_apply_shape64(p, sh);
+        if (int e = plan_apply_shape64(p, sh))
+            return e;
+    } else {
+        const FourStep* sh = find_shape(p->lg, n2_log2, rows, cols);
+        if (!sh)
+            return fail(PCX_ERR_UNSUPPORTED, "no four-step shape of fft_size " + s(p->n) + " matches");
+        if (int e = plan_apply_shape(p, sh))
+            return e;
     }
-    const FourStep* sh = find_shape(p->lg, n2_log2, rows, cols);
-    if (!sh)
-        return fail(PCX_ERR_UNSUPPORTED, "no four-step shape of fft_size " + s(p->n) + " matches");
-    return plan_apply_shape(p, sh);
+    p->auto_shape = n2_log2 == 0 && cols == 0 && rows == 0;
+    return PCX_SUCCESS;
 }
 
 extern "C" int pcx_plan_shape(pcx_plan_t p, int* n2_log2, int* cols, int* rows) {
@@ -840,9 +893,9 @@ extern "C" int pcx_plan_set_three_pass(pcx_plan_t p, int enable) {
 extern "C" int pcx_plan_set_one_pass(pcx_plan_t p, int enable) {
     if (!p)
         return fail(PCX_ERR_INVALID_ARGUMENT, "plan is null");
-    if (!p->tw_dif)
+    if (!p->tw_one || p->f64)
         return enable ? fail(PCX_ERR_UNSUPPORTED, "no one-pass kernel for fft_size " + s(p->n)) : PCX_SUCCESS;
-    p->use_dif = enable != 0;
+    p->use_one = enable != 0;
     return PCX_SUCCESS;
 }
 
@@ -1761,6 +1814,7 @@ extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, v
                                     return err;
                                 }
                                 g.plan->grid_col = gc, g.plan->grid_row = gr;
+                                g.plan->auto_shape = false;
                             }
                         }
                 } else {
@@ -1836,6 +1890,7 @@ extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, v
         const FourStep* best = g.plan->shape;
         int64_t         bgc = g.plan->grid_col, bgr = g.plan->grid_row;
         float           bms = 1e30f;
+        g.plan->auto_shape = false; // the candidates themselves are timed
         std::vector<const FourStep*> cands;
         for (const ShapeList<float>& l : {shapes_default(), shapes_alt()})
             for (int i = 0; i < l.count; ++i)

@@ -23,7 +23,8 @@ constexpr std::array<ColLaunch, 2> col_set() {
 template<int LG, int N1, int N2, int G, int C, int PXC = 0>
 constexpr FourStep shape() {
     static_assert(N1 + N2 == LG, "shape");
-    return {LG, N1, N2, G, C, pass_set<N1, G, LG>(), col_set<N2, C, LG, PXC>()};
+    return {LG, N1, N2, G, C, pass_set<N1, G, LG>(), col_set<N2, C, LG, PXC>(),
+            (G << N1) >= 16384 || (C << N2) >= 16384 ? kWideGrid : 0};
 }
 
 // FP64 shapes, 256-512 threads per workgroup.  C and G are the doubles per column segment and
@@ -38,7 +39,8 @@ constexpr FourStepT<double> shape64() {
              &launch_row<N1, G, LD_CONTIG, ST_PERM, 0, true, ORD_BITREV, PREC_FP32, D>, nullptr,
              &launch_row<N1, G, LD_STRIDED, ST_CONTIG, TW, true, 0, PREC_FP32, D>,
              &launch_row<N1, G, LD_PERM, ST_CONTIG, TW, true, ORD_BITREV, PREC_FP32, D>, nullptr},
-            {&launch_col<N2, C, 0, PREC_FP32, D>, &launch_col<N2, C, TW, PREC_FP32, D>}};
+            {&launch_col<N2, C, 0, PREC_FP32, D>, &launch_col<N2, C, TW, PREC_FP32, D>},
+            (G << N1) >= 8192 || (C << N2) >= 8192 ? kWideGrid : 0};
 }
 
 } // namespace pcxd
