@@ -59,9 +59,7 @@ void launch_across(const AcrossArgsT<T>& a, int64_t grid, hipStream_t st) {
     constexpr int C  = across_cols<LA, T>();
     constexpr int NT = C * Plan<LA, false, T>::TA;
     static_assert(NT <= 1024, "across tile");
-    int64_t n = (a.len + C - 1) / C;
-    if (n > grid)
-        n = grid;
+    const int64_t n = even_grid((a.len + C - 1) / C, grid);
     hipLaunchKernelGGL((k_across<LA, C, T>), dim3((unsigned)fit_grid(grid8(n), NT)), dim3(NT), 0, st, a);
 }
 template<class T, int... L>

@@ -634,7 +634,7 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
 
     // ---- one pass, radix-R decimation in frequency + M-point Stockham (no intermediate)
     if constexpr (!F64)
-    if (p->use_one && p->precision == PCX_PREC_FP32 && batch >= kDifBatch && (const float*)dst != src &&
+    if (p->use_one && p->precision == PCX_PREC_FP32 && batch >= kDifBatch && (const float*)dst != src && !src_offs &&
         (!inverse || p->order == PCX_ORDER_NORMAL)) {
         RowArgs a{};
         a.src = src, a.dst = dst, a.src_dist = src_dist, a.dst_dist = dst_dist;
@@ -1421,13 +1421,13 @@ extern "C" int pcx_generate_f64(double* dst, int64_t pack, int64_t n, uint64_t s
 // ---------------------------------------------------------------- uneven-batch work queue
 namespace {
 
-struct QGroup { // transforms of one size above 2^20 and one direction: grouped four-step launches
-    int      lg   = 0;
-    int      inv  = 0;
-    int64_t  count = 0;
-    int64_t* src_offs = nullptr; // device
-    int64_t* dst_offs = nullptr;
-    pcx_plan_t plan = nullptr;
+struct QGroup { // transforms of one size and one direction that run as full-chip launches
+    int        lg    = 0;
+    int        inv   = 0;
+    int64_t    count = 0;
+    int64_t    first = 0; // index of the first one in the offset tables
+    pcx_plan_t plan  = nullptr;
+    bool       own   = false; // the plan is this group's (else the other direction's)
 };
 
 } // namespace
@@ -1436,23 +1436,26 @@ struct pcx_queue_s {
     int                 normalized = 1;
     int64_t             njobs      = 0;
     double              flops = 0, bytes = 0;
-    // persistent part: every transform of 2^1 .. 2^20 points
+    // persistent part: transforms of 2^1 .. 2^14 points
     int32_t             nitems     = 0;
     QItem*              items      = nullptr; // device
-    int64_t*            q_src_offs = nullptr;
-    int64_t*            q_dst_offs = nullptr;
-    uint32_t*           counter    = nullptr;
+    int64_t*            src_offs   = nullptr; // per transform: items first, then the groups
+    int64_t*            dst_offs   = nullptr;
     float2*             tw         = nullptr; // W_A for A = 2 .. 2^14
-    float2*             ptw        = nullptr; // pass tables of 2^15 .. 2^20
-    int32_t             ptw_off[kQueueMaxLog2 + 1] = {};
-    float*              tmp        = nullptr; // four-step intermediates, one per workgroup
-    int64_t             tmp_floats = 0;
     int                 grid       = 0;       // workgroups of the persistent launch
-    int                 grid_cap   = 0;       // workgroups the intermediates were sized for
-    // grouped part: sizes above 2^20, and the classes the autotuner moved out of the persistent
-    // launch (grouped[log2n][inverse])
+    int                 grid_cap   = 0;
+    // grouped part, largest size first: sizes above 2^14, and the classes the autotuner moved out of
+    // the persistent launch (grouped[log2n][inverse]); the groups run one after another through
+    // one four-step intermediate
     std::vector<QGroup> groups;
-    bool                grouped[kMaxLog2 + 1][2] = {};
+    void*               tmp        = nullptr;
+    int64_t             tmp_bytes  = 0;
+    // a call on another stream than the intermediate's last user waits for that use
+    hipEvent_t          tmp_ev     = nullptr;
+    hipStream_t         tmp_stream = nullptr;
+    bool                tmp_used   = false;
+    std::mutex          mu;
+    bool                grouped[kQueueMaxLog2 + 1][2] = {};
     std::vector<pcx_job> jobs; // the job list, to rebuild the items when the split changes
     // captured graph
     hipGraph_t          graph = nullptr;
@@ -1461,23 +1464,41 @@ struct pcx_queue_s {
 
 namespace {
 
+int queue_run_group(pcx_queue_t q, const QGroup& g, float* dst, const float* src, hipStream_t st) {
+    const int64_t n = (int64_t)1 << g.lg;
+    const ExtTmp  ext{q->tmp, q->tmp_bytes};
+    return run_batch(g.plan, g.inv, q->normalized, dst, n, 2 * n, src, n, 2 * n, n, g.count, st, q->src_offs + g.first,
+                     q->dst_offs + g.first, &ext);
+}
+
 int queue_run(pcx_queue_t q, float* dst, const float* src, hipStream_t st) {
     if (q->nitems > 0) {
-        launch_reset_counter(q->counter, st);
         QueueArgs a{};
-        a.src = src, a.dst = dst, a.tmp = q->tmp, a.tmp_floats = q->tmp_floats;
-        a.src_offs = q->q_src_offs, a.dst_offs = q->q_dst_offs;
-        a.items = q->items, a.nitems = q->nitems, a.normalized = q->normalized, a.counter = q->counter;
-        a.tw = q->tw, a.ptw = q->ptw;
-        std::memcpy(a.ptw_off, q->ptw_off, sizeof(a.ptw_off));
+        a.src = src, a.dst = dst;
+        a.src_offs = q->src_offs, a.dst_offs = q->dst_offs;
+        a.items = q->items, a.nitems = q->nitems, a.normalized = q->normalized;
+        a.tw = q->tw;
         launch_queue(a, std::min<int>(q->grid, q->nitems), st);
         HIPCHK(hipGetLastError());
     }
-    for (auto& g : q->groups) {
-        int64_t n = (int64_t)1 << g.lg;
-        if (int e = run_batch(g.plan, g.inv, q->normalized, dst, n, 2 * n, src, n, 2 * n, n, g.count, st, g.src_offs,
-                              g.dst_offs))
+    if (!q->tmp) {
+        for (const auto& g : q->groups)
+            if (int e = queue_run_group(q, g, dst, src, st))
+                return e;
+        return PCX_SUCCESS;
+    }
+    std::lock_guard<std::mutex> lock(q->mu);
+    hipStreamCaptureStatus      cs = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(st, &cs));
+    const bool capturing = cs != hipStreamCaptureStatusNone;
+    if (q->tmp_used && q->tmp_stream != st && !capturing)
+        HIPCHK(hipStreamWaitEvent(st, q->tmp_ev, 0));
+    for (const auto& g : q->groups)
+        if (int e = queue_run_group(q, g, dst, src, st))
             return e;
+    if (!capturing) {
+        HIPCHK(hipEventRecord(q->tmp_ev, st));
+        q->tmp_stream = st, q->tmp_used = true;
     }
     return PCX_SUCCESS;
 }
@@ -1489,20 +1510,21 @@ void queue_release(pcx_queue_t q) {
     if (q->graph)
         (void)hipGraphDestroy(q->graph);
     q->exec = nullptr, q->graph = nullptr;
+    if (q->tmp_ev && q->tmp_used)
+        (void)hipEventSynchronize(q->tmp_ev);
+    if (q->tmp_ev)
+        (void)hipEventDestroy(q->tmp_ev);
+    q->tmp_ev = nullptr, q->tmp_used = false;
     (void)hipFree(q->items);
-    (void)hipFree(q->q_src_offs);
-    (void)hipFree(q->q_dst_offs);
-    (void)hipFree(q->counter);
+    (void)hipFree(q->src_offs);
+    (void)hipFree(q->dst_offs);
     (void)hipFree(q->tw);
-    (void)hipFree(q->ptw);
     (void)hipFree(q->tmp);
-    q->items = nullptr, q->q_src_offs = q->q_dst_offs = nullptr, q->counter = nullptr;
-    q->tw = q->ptw = nullptr, q->tmp = nullptr, q->tmp_floats = 0, q->nitems = 0;
-    for (auto& g : q->groups) {
-        (void)hipFree(g.src_offs);
-        (void)hipFree(g.dst_offs);
-        pcx_plan_destroy(g.plan);
-    }
+    q->items = nullptr, q->src_offs = q->dst_offs = nullptr, q->tw = nullptr, q->nitems = 0;
+    q->tmp = nullptr, q->tmp_bytes = 0;
+    for (auto& g : q->groups)
+        if (g.own)
+            pcx_plan_destroy(g.plan);
     q->groups.clear();
 }
 
@@ -1511,8 +1533,8 @@ void queue_free(pcx_queue_t q) {
     delete q;
 }
 
-// Builds the persistent items (every class up to 2^20 not marked grouped, largest first) and the
-// grouped launches (the rest, largest first) from the job list.
+// Builds the persistent items (every class up to 2^14 not marked grouped) and the grouped launches
+// (the rest), both largest first, from the job list.
 int queue_build(pcx_queue_t q) {
     const pcx_job* jobs  = q->jobs.data();
     const int64_t  njobs = (int64_t)q->jobs.size();
@@ -1521,96 +1543,79 @@ int queue_build(pcx_queue_t q) {
         bucket[jobs[i].log2n * 2 + jobs[i].inverse].push_back(i);
     std::vector<QItem>   items;
     std::vector<int64_t> qs, qd;
-    int                  max_four = 0;
-    // persistent items, largest size first (longest-processing-time order)
+    auto                 put = [&](int64_t job) {
+        qs.push_back(jobs[job].src_offset);
+        qd.push_back(jobs[job].dst_offset);
+    };
     for (int lg = kQueueMaxLog2; lg >= 1; --lg) {
-        const int per = lg >= kQueueMinFour ? 1 : kQueueThreads / (lg >= 4 ? (1 << lg) / 16 : 1);
+        const int per = std::max(1, kQueueThreads / (lg >= 4 ? (1 << lg) / 16 : 1));
         for (int inv = 0; inv < 2; ++inv) {
             if (q->grouped[lg][inv])
                 continue;
             auto& b = bucket[lg * 2 + inv];
             for (size_t k = 0; k < b.size(); k += per) {
                 int cnt = (int)std::min<size_t>(per, b.size() - k);
-                items.push_back({lg >= kQueueMinFour ? QK_FOUR : QK_SINGLE, lg, inv, (int32_t)qs.size(), cnt});
-                for (int c = 0; c < cnt; ++c) {
-                    qs.push_back(jobs[b[k + c]].src_offset);
-                    qd.push_back(jobs[b[k + c]].dst_offset);
-                }
-                if (lg >= kQueueMinFour)
-                    max_four = std::max(max_four, lg);
+                items.push_back({lg, inv, (int32_t)qs.size(), cnt});
+                for (int c = 0; c < cnt; ++c)
+                    put(b[k + c]);
             }
         }
     }
     q->nitems = (int32_t)items.size();
-    hipStream_t setup = nullptr;
-    hipError_t  he    = setup_stream(&setup);
-    if (!items.empty() && he == hipSuccess) {
-        he = hipMalloc(&q->items, sizeof(QItem) * items.size());
-        if (he == hipSuccess)
-            he = hipMalloc(&q->q_src_offs, sizeof(int64_t) * qs.size());
-        if (he == hipSuccess)
-            he = hipMalloc(&q->q_dst_offs, sizeof(int64_t) * qd.size());
-        if (he == hipSuccess)
-            he = hipMalloc(&q->counter, sizeof(uint32_t));
-        if (he == hipSuccess)
-            he = hipMalloc(&q->tw, sizeof(float2) * ((1 << (kQueueMaxSingle + 1)) - 2));
-        if (he == hipSuccess)
-            he = hipMemcpy(q->items, items.data(), sizeof(QItem) * items.size(), hipMemcpyHostToDevice);
-        if (he == hipSuccess)
-            he = hipMemcpy(q->q_src_offs, qs.data(), sizeof(int64_t) * qs.size(), hipMemcpyHostToDevice);
-        if (he == hipSuccess)
-            he = hipMemcpy(q->q_dst_offs, qd.data(), sizeof(int64_t) * qd.size(), hipMemcpyHostToDevice);
-        for (int lg = 1; lg <= kQueueMaxSingle && he == hipSuccess; ++lg)
-            he = gen_twiddles(q->tw + ((1 << lg) - 2), (int64_t)1 << lg, 1, (int64_t)1 << lg, setup);
-        if (max_four > 0 && he == hipSuccess) {
-            // pass tables W_N^e = lo[e mod 2^ls] * hi[e >> ls] of every four-step size, and one
-            // intermediate of the largest size per workgroup
-            int64_t total = 0;
-            for (int lg = kQueueMinFour; lg <= max_four; ++lg) {
-                q->ptw_off[lg] = (int32_t)total;
-                total += ((int64_t)1 << ((lg + 1) / 2)) + ((int64_t)1 << (lg - (lg + 1) / 2));
-            }
-            he = hipMalloc(&q->ptw, sizeof(float2) * total);
-            for (int lg = kQueueMinFour; lg <= max_four && he == hipSuccess; ++lg) {
-                const int     ls = (lg + 1) / 2;
-                const int64_t nl = (int64_t)1 << ls, nh = ((int64_t)1 << lg) >> ls;
-                he = gen_twiddles(q->ptw + q->ptw_off[lg], (int64_t)1 << lg, 1, nl, setup);
-                if (he == hipSuccess)
-                    he = gen_twiddles(q->ptw + q->ptw_off[lg] + nl, (int64_t)1 << lg, nl, nh, setup);
-            }
-            q->tmp_floats = (int64_t)2 << max_four;
-            if (he == hipSuccess)
-                he = hipMalloc(&q->tmp, sizeof(float) * q->tmp_floats * q->grid_cap);
-        }
-    }
-    // grouped launches, largest first
-    for (int lg = kMaxLog2; lg >= 1 && he == hipSuccess; --lg) {
+    for (int lg = kMaxLog2; lg >= 1; --lg)
         for (int inv = 0; inv < 2; ++inv) {
             auto& b = bucket[lg * 2 + inv];
             if (b.empty() || (lg <= kQueueMaxLog2 && !q->grouped[lg][inv]))
                 continue;
             QGroup g;
-            g.lg = lg, g.inv = inv, g.count = (int64_t)b.size();
-            std::vector<int64_t> so(b.size()), dof(b.size());
-            for (size_t k = 0; k < b.size(); ++k)
-                so[k] = jobs[b[k]].src_offset, dof[k] = jobs[b[k]].dst_offset;
-            he = hipMalloc(&g.src_offs, sizeof(int64_t) * b.size());
-            if (he == hipSuccess)
-                he = hipMalloc(&g.dst_offs, sizeof(int64_t) * b.size());
-            if (he == hipSuccess)
-                he = hipMemcpy(g.src_offs, so.data(), sizeof(int64_t) * b.size(), hipMemcpyHostToDevice);
-            if (he == hipSuccess)
-                he = hipMemcpy(g.dst_offs, dof.data(), sizeof(int64_t) * b.size(), hipMemcpyHostToDevice);
+            g.lg = lg, g.inv = inv, g.count = (int64_t)b.size(), g.first = (int64_t)qs.size();
+            for (int64_t job : b)
+                put(job);
+            // both directions of a size share a plan (until they are tuned)
+            g.own = q->groups.empty() || q->groups.back().lg != lg;
+            if (!g.own)
+                g.plan = q->groups.back().plan;
+            else if (int e = pcx_plan_create((int64_t)1 << lg, 2048, PCX_ORDER_NORMAL, &g.plan))
+                return e;
             q->groups.push_back(g);
-            if (he == hipSuccess)
-                if (int e = pcx_plan_create((int64_t)1 << lg, 2048, PCX_ORDER_NORMAL, &q->groups.back().plan))
-                    return e;
+            if (lg > kQueueMaxLog2)
+                q->tmp_bytes = std::max(q->tmp_bytes, std::min(g.count, g.plan->chunk) * 8 * g.plan->n);
         }
+    hipStream_t setup = nullptr;
+    hipError_t  he    = setup_stream(&setup);
+    auto        upload = [&](auto** dev, const auto& v) {
+        if (v.empty() || he != hipSuccess)
+            return;
+        he = hipMalloc(dev, sizeof(v[0]) * v.size());
+        if (he == hipSuccess)
+            he = hipMemcpy(*dev, v.data(), sizeof(v[0]) * v.size(), hipMemcpyHostToDevice);
+    };
+    upload(&q->items, items);
+    upload(&q->src_offs, qs);
+    upload(&q->dst_offs, qd);
+    if (q->tmp_bytes > 0 && he == hipSuccess)
+        he = hipMalloc(&q->tmp, q->tmp_bytes);
+    if (q->tmp_bytes > 0 && he == hipSuccess)
+        he = hipEventCreateWithFlags(&q->tmp_ev, hipEventDisableTiming);
+    if (!items.empty() && he == hipSuccess) {
+        he = hipMalloc(&q->tw, sizeof(float2) * ((1 << (kQueueMaxLog2 + 1)) - 2));
+        for (int lg = 1; lg <= kQueueMaxLog2 && he == hipSuccess; ++lg)
+            he = gen_twiddles(q->tw + ((1 << lg) - 2), (int64_t)1 << lg, 1, (int64_t)1 << lg, setup);
+        if (he == hipSuccess)
+            he = hipStreamSynchronize(setup);
     }
-    if (he == hipSuccess)
-        he = hipStreamSynchronize(setup);
     if (he != hipSuccess)
         return fail(PCX_ERR_HIP, std::string("queue setup: ") + hipGetErrorString(he));
+    return PCX_SUCCESS;
+}
+
+// Gives a group a plan of its own, so that tuning it leaves the other direction's alone.
+int queue_own_plan(QGroup& g) {
+    if (g.own)
+        return PCX_SUCCESS;
+    if (int e = pcx_plan_create((int64_t)1 << g.lg, 2048, PCX_ORDER_NORMAL, &g.plan))
+        return e;
+    g.own = true;
     return PCX_SUCCESS;
 }
 
@@ -1636,8 +1641,8 @@ extern "C" int pcx_queue_create(const pcx_job* jobs, int64_t njobs, int normaliz
     auto* q       = new pcx_queue_s;
     q->normalized = normalized ? 1 : 0;
     q->njobs      = njobs;
-    // one workgroup per CU (the largest item takes most of a CU's LDS); the autotuner may pick fewer
-    q->grid = q->grid_cap = std::max(1, ncu);
+    // two workgroups per CU; the autotuner may pick fewer
+    q->grid = q->grid_cap = 2 * std::max(1, ncu);
     for (int64_t i = 0; i < njobs; ++i) {
         double n = (double)((int64_t)1 << jobs[i].log2n);
         q->flops += 5.0 * n * (double)jobs[i].log2n;
@@ -1674,15 +1679,6 @@ extern "C" int pcx_queue_capture(pcx_queue_t q, float* dst, const float* src, vo
     hipStream_t st = (hipStream_t)stream;
     if (!st)
         return fail(PCX_ERR_INVALID_ARGUMENT, "graph capture needs a non-default stream");
-    // make sure every group's intermediate exists before capture (allocation is not capturable)
-    for (auto& g : q->groups) {
-        int64_t n = (int64_t)1 << g.lg;
-        if (g.plan->two_pass && g.plan->tmp_cap < std::min(g.count, g.plan->chunk)) {
-            if (int e = run_batch(g.plan, g.inv, q->normalized, dst, n, 2 * n, src, n, 2 * n, n, g.count, st,
-                                  g.src_offs, g.dst_offs))
-                return e;
-        }
-    }
     HIPCHK(hipStreamSynchronize(st));
     if (q->exec) {
         HIPCHK(hipGraphExecDestroy(q->exec));
@@ -1784,7 +1780,7 @@ extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, v
             int  a = 0, b = 0, c = 0, d = 0, e = 0;
             long long gc = 0, gr = 0;
             // the split between the persistent launch and grouped launches comes first
-            bool mask[kMaxLog2 + 1][2] = {};
+            bool mask[kQueueMaxLog2 + 1][2] = {};
             long pos = std::ftell(f);
             while (std::fscanf(f, "%31s", key) == 1) {
                 if (!std::strcmp(key, "grouped") && std::fscanf(f, "%d %d", &a, &b) == 2 && a >= 1 && a <= kQueueMaxLog2 &&
@@ -1809,12 +1805,16 @@ extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, v
                     for (auto& g : q->groups)
                         if (g.lg == a && g.inv == b && g.plan->two_pass) {
                             if (const FourStep* sh = find_shape(a, c, d, e)) {
-                                if (int err = plan_apply_shape(g.plan, sh)) {
+                                int err = queue_own_plan(g);
+                                if (!err)
+                                    err = plan_apply_shape(g.plan, sh);
+                                if (err) {
                                     std::fclose(f);
                                     return err;
                                 }
+                                // grid caps of -1: the plan's own choice of shape and caps won
                                 g.plan->grid_col = gc, g.plan->grid_row = gr;
-                                g.plan->auto_shape = false;
+                                g.plan->auto_shape = gc < 0;
                             }
                         }
                 } else {
@@ -1844,75 +1844,62 @@ extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, v
         }
         q->grid = bg;
     }
-    // which size classes run in the persistent launch and which as grouped launches after it:
-    // each four-step class (largest first), then the single-pass classes together, moves out when
-    // that makes the whole pass faster
+    // the sizes of the persistent launch move out to grouped launches when that makes the whole pass
+    // faster
     {
-        bool present[kMaxLog2 + 1] = {};
+        bool present[kQueueMaxLog2 + 1] = {}, any = false;
         for (const auto& j : q->jobs)
-            present[j.log2n] = true;
-        auto whole = [&] { return queue_run(q, dst, src, st); };
+            if (j.log2n <= kQueueMaxLog2)
+                present[j.log2n] = any = true;
+        auto whole   = [&] { return queue_run(q, dst, src, st); };
         auto rebuild = [&]() -> int {
             queue_release(q);
             return queue_build(q);
         };
-        float best = time_ms(st, whole);
-        auto  trial = [&](int lo, int hi) -> int {
-            bool any = false;
-            for (int lg = lo; lg <= hi; ++lg)
-                any = any || (present[lg] && !q->grouped[lg][0]);
-            if (!any)
-                return PCX_SUCCESS;
-            bool keep[kMaxLog2 + 1][2];
-            std::memcpy(keep, q->grouped, sizeof(keep));
-            for (int lg = lo; lg <= hi; ++lg)
+        if (any) {
+            const float best = time_ms(st, whole);
+            for (int lg = 1; lg <= kQueueMaxLog2; ++lg)
                 q->grouped[lg][0] = q->grouped[lg][1] = present[lg];
             if (int e = rebuild())
                 return e;
-            const float ms = time_ms(st, whole);
-            if (ms < best) {
-                best = ms;
-                return PCX_SUCCESS;
+            if (!(time_ms(st, whole) < best)) {
+                std::memset(q->grouped, 0, sizeof(q->grouped));
+                if (int e = rebuild())
+                    return e;
             }
-            std::memcpy(q->grouped, keep, sizeof(keep));
-            return rebuild();
-        };
-        for (int lg = kQueueMaxLog2; lg >= kQueueMinFour; --lg)
-            if (int e = trial(lg, lg))
-                return e;
-        if (int e = trial(1, kQueueMaxSingle))
-            return e;
+        }
     }
     for (auto& g : q->groups) {
         if (!g.plan->two_pass)
             continue;
-        int64_t         n    = (int64_t)1 << g.lg;
-        const FourStep* best = g.plan->shape;
-        int64_t         bgc = g.plan->grid_col, bgr = g.plan->grid_row;
-        float           bms = 1e30f;
-        g.plan->auto_shape = false; // the candidates themselves are timed
+        if (int err = queue_own_plan(g))
+            return err;
+        pcx_plan_t      p    = g.plan;
+        auto            time = [&] { return time_ms(st, [&] { return queue_run_group(q, g, dst, src, st); }); };
+        // the plan's own choice first (grid caps -1), then every instantiated shape and cap
+        const FourStep* best = p->shape;
+        int64_t         bgc  = -1;
+        float           bms  = time();
         std::vector<const FourStep*> cands;
         for (const ShapeList<float>& l : {shapes_default(), shapes_alt()})
             for (int i = 0; i < l.count; ++i)
                 if (l.data[i].lg == g.lg)
                     cands.push_back(&l.data[i]);
-        for (const FourStep* shp : cands) {
-            const FourStep& sh = *shp;
-            if (int err = plan_apply_shape(g.plan, &sh))
+        p->auto_shape = false;
+        for (const FourStep* sh : cands) {
+            if (int err = plan_apply_shape(p, sh))
                 return err;
             for (int64_t gc : {(int64_t)0, (int64_t)1024, (int64_t)2048}) {
-                g.plan->grid_col = g.plan->grid_row = gc;
-                float ms = time_ms(st, [&] {
-                    return run_batch(g.plan, g.inv, q->normalized, dst, n, 2 * n, src, n, 2 * n, n, g.count, st,
-                                     g.src_offs, g.dst_offs);
-                });
+                p->grid_col = p->grid_row = gc;
+                const float ms = time();
                 if (ms < bms)
-                    bms = ms, best = &sh, bgc = gc, bgr = gc;
+                    bms = ms, best = sh, bgc = gc;
             }
         }
-        if (int err = plan_apply_shape(g.plan, best))
+        if (int err = plan_apply_shape(p, best))
             return err;
-        g.plan->grid_col = bgc, g.plan->grid_row = bgr;
+        p->grid_col = p->grid_row = bgc;
+        p->auto_shape = bgc < 0;
     }
     if (cache_path) {
         if (FILE* f = std::fopen(cache_path, "w")) {
