@@ -115,9 +115,9 @@ SIGNATURES = {
     "pcx_synchronize": (_int, [_vp]),
     "pcx_generate": (_int, [_vp, _i64, _i64, _u64, _int, _dbl, _vp]),
     "pcx_generate_f64": (_int, [_vp, _i64, _i64, _u64, _int, _dbl, _vp]),
-    "pcx_vexpr_eval": (_int, [C.POINTER(VSource), C.c_int32, C.POINTER(VInstr), C.c_int32, _vp, _i64, _i64, _vp]),
+    "pcx_vexpr_eval": (_int, [_vp, C.c_int32, _vp, C.c_int32, _vp, _i64, _i64, _vp]),
     "pcx_repack": (_int, [_vp, _i64, _vp, _i64, _i64, _vp]),
-    "pcx_vexpr_eval_f64": (_int, [C.POINTER(VSource64), C.c_int32, C.POINTER(VInstr64), C.c_int32, _vp, _i64, _i64,
+    "pcx_vexpr_eval_f64": (_int, [_vp, C.c_int32, _vp, C.c_int32, _vp, _i64, _i64,
                                   _vp]),
     "pcx_repack_f64": (_int, [_vp, _i64, _vp, _i64, _i64, _vp]),
     "pcx_fft_across": (_int, [_vp, _int, _int, _vp, _i64, _vp, _i64, _i64, _vp]),
@@ -125,6 +125,27 @@ SIGNATURES = {
 }
 
 _lib = None
+_raw_stream = None
+
+
+def _current_stream():
+    global _raw_stream
+    import torch
+
+    if not torch.cuda.is_available():
+        raise RuntimeError("packed_amd needs a ROCm GPU: torch.cuda.is_available() is False")
+    torch.cuda.current_stream()  # initialises the runtime
+    get, dev = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+    _raw_stream = lambda: get(dev())  # noqa: E731
+    return _raw_stream()
+
+
+def stream_ptr(stream):
+    """hipStream_t of a torch stream, a raw handle, or (None) torch's current stream: looked up by
+    every call, without building a torch.cuda.Stream object for it (0.3 against 3.2 us)."""
+    if stream is None:
+        return (_raw_stream or _current_stream)()
+    return getattr(stream, "cuda_stream", stream)
 
 
 class PcxError(ValueError):

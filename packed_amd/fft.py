@@ -19,6 +19,8 @@ import numpy as np
 
 from . import _lib
 from ._lib import ORDER, PRECISION, PcxError, check, lib
+from ._lib import stream_ptr as _stream_ptr
+from .vexpr import Leaf
 
 __all__ = ["vector", "md_storage", "fft_unit", "fxcorr_unit", "fft_queue", "PcxError", "real_size", "pidx"]
 
@@ -40,13 +42,6 @@ def pidx(i, pack: int):
     """element_access.hpp:8-11: float offset of the real part of complex i."""
     i = np.asarray(i, dtype=np.int64)
     return i + (i // pack) * pack
-
-
-def _stream_ptr(stream) -> int | None:
-    if stream is None:
-        torch = _torch()
-        return torch.cuda.current_stream().cuda_stream
-    return getattr(stream, "cuda_stream", stream)
 
 
 DTYPES = ("float32", "float64")
@@ -99,8 +94,6 @@ class vector:
 
     # vector_arithm.hpp:450-495: lazy expressions, evaluated on the GPU by store()
     def _expr(self):
-        from .vexpr import Leaf
-
         return Leaf(self)
 
     def __add__(self, o):
@@ -198,6 +191,7 @@ class fft_unit:
         create = lib().pcx_plan_create_f64 if dtype == "float64" else lib().pcx_plan_create
         check(create(int(fft_size), int(sub_size), ORDER[order], C.byref(h)))
         self._h = h
+        self._n = int(fft_size)
         self.order = order
         self.dtype = dtype
         f64 = dtype == "float64"
@@ -219,7 +213,7 @@ class fft_unit:
         return self._h
 
     def size(self) -> int:
-        return int(lib().pcx_plan_size(self._h))
+        return self._n
 
     # ---------------------------------------------------------------- launch-shape tuning
     def set_shape(self, n2_log2: int = 0, cols: int = 0, rows: int = 0) -> None:
@@ -339,36 +333,42 @@ class fft_unit:
         if isinstance(dst, md_storage):
             self._storage_call(dst, src, False, True, stream)
             return
-        self._check_type(dst, *([] if src is None else [src]))
+        n = self._n
         if src is None:
-            if dst.size() != self.size():
+            self._check_type(dst)
+            if dst.size() != n:
                 raise PcxError(_lib.ERR_SIZE_MISMATCH, f"input size (which is {dst.size()}) is not equal to fft "
-                                                       f"size (which is {self.size()})")
-            self.fft_raw(dst.data_ptr(), dst.data_ptr(), dst.pack, dst.pack, self.size(), stream)
+                                                       f"size (which is {n})")
+            ptr = dst.data_ptr()
+            check(self._fft(self._h, ptr, dst.pack, ptr, dst.pack, n, _stream_ptr(stream)))
             return
+        self._check_type(dst, src)
         self._check_dst(dst, "destination")
-        if src.size() > self.size():
+        if src.size() > n:
             raise PcxError(_lib.ERR_SIZE_MISMATCH, f"source size (which is {src.size()}) is bigger than fft size "
-                                                   f"(which is {self.size()})")
-        self.fft_raw(dst.data_ptr(), src.data_ptr(), dst.pack, src.pack, src.size(), stream)
+                                                   f"(which is {n})")
+        check(self._fft(self._h, dst.data_ptr(), dst.pack, src.data_ptr(), src.pack, src.size(), _stream_ptr(stream)))
 
     def ifft(self, dst: vector, src: vector | None = None, normalized: bool = True, stream=None) -> None:
         """ifft<Normalized>(v) / ifft<Normalized>(dst, src) (fft.hpp:828-915); md_storage: every slice."""
         if isinstance(dst, md_storage):
             self._storage_call(dst, src, True, normalized, stream)
             return
-        self._check_type(dst, *([] if src is None else [src]))
+        n = self._n
         if src is None:
-            if dst.size() != self.size():
+            self._check_type(dst)
+            if dst.size() != n:
                 raise PcxError(_lib.ERR_SIZE_MISMATCH, f"input size (which is {dst.size()} is not equal to fft "
-                                                       f"size (which is {self.size()})")
+                                                       f"size (which is {n})")
             src = dst
         else:
+            self._check_type(dst, src)
             self._check_dst(dst, "destination")
-            if src.size() != self.size():
+            if src.size() != n:
                 raise PcxError(_lib.ERR_SIZE_MISMATCH, f"source size (which is {src.size()}) is not equal to fft "
-                                                       f"size (which is {self.size()})")
-        self.ifft_raw(dst.data_ptr(), src.data_ptr(), normalized, dst.pack, src.pack, stream)
+                                                       f"size (which is {n})")
+        check(self._ifft(self._h, int(normalized), dst.data_ptr(), dst.pack, src.data_ptr(), src.pack,
+                         _stream_ptr(stream)))
 
 
 class fxcorr_unit:

@@ -13,9 +13,10 @@ The machine has four registers, so any expression whose tree needs at most four 
 from __future__ import annotations
 
 import numbers
+import struct
 
 from . import _lib
-from ._lib import PcxError, check, lib
+from ._lib import PcxError, check, lib, stream_ptr
 
 _BIN = {"+": "ADD", "-": "SUB", "*": "MUL", "/": "DIV"}
 # scalar ops: (op with scalar on the right, op with scalar on the left); real and complex forms
@@ -24,6 +25,8 @@ _SCA = {"+": ("ADD", "ADD"), "-": ("SUB", "RSUB"), "*": ("MUL", "MUL"), "/": ("D
 
 class Expr:
     """A lazy element-wise expression over packed device vectors."""
+
+    __slots__ = ()
 
     def __add__(self, o):
         return _combine("+", self, o)
@@ -49,58 +52,47 @@ class Expr:
     def __rtruediv__(self, o):
         return _combine("/", o, self)
 
+    # n: elements; regs: registers its evaluation needs (set when a node is built)
     def size(self) -> int:
-        raise NotImplementedError
+        return self.n
 
     def need(self) -> int:
-        raise NotImplementedError
+        return self.regs
 
 
 class Leaf(Expr):
+    __slots__ = ("vec", "n", "regs")
+
     def __init__(self, vec):
         self.vec = vec
-
-    def size(self):
-        return self.vec.size()
-
-    def need(self):
-        return 1
+        self.n, self.regs = vec.size(), 1
 
 
 class Bin(Expr):
+    __slots__ = ("op", "lhs", "rhs", "n", "regs")
+
     def __init__(self, op, lhs, rhs):
-        if lhs.size() != rhs.size():
-            raise PcxError(_lib.ERR_SIZE_MISMATCH, f"vector sizes {lhs.size()} and {rhs.size()} differ")
+        if lhs.n != rhs.n:
+            raise PcxError(_lib.ERR_SIZE_MISMATCH, f"vector sizes {lhs.n} and {rhs.n} differ")
         self.op, self.lhs, self.rhs = op, lhs, rhs
-
-    def size(self):
-        return self.lhs.size()
-
-    def need(self):
-        a, b = self.lhs.need(), self.rhs.need()
-        return max(a, b) if a != b else a + 1
+        self.n = lhs.n
+        self.regs = max(lhs.regs, rhs.regs) if lhs.regs != rhs.regs else lhs.regs + 1
 
 
 class Scalar(Expr):
+    __slots__ = ("op", "expr", "scalar", "left", "n", "regs")
+
     def __init__(self, op, expr, scalar, scalar_left):
         self.op, self.expr, self.scalar, self.left = op, expr, scalar, scalar_left
-
-    def size(self):
-        return self.expr.size()
-
-    def need(self):
-        return self.expr.need()
+        self.n, self.regs = expr.n, expr.regs
 
 
 class Conj(Expr):
+    __slots__ = ("expr", "n", "regs")
+
     def __init__(self, expr):
         self.expr = expr
-
-    def size(self):
-        return self.expr.size()
-
-    def need(self):
-        return self.expr.need()
+        self.n, self.regs = expr.n, expr.regs
 
 
 def as_expr(x) -> Expr:
@@ -111,9 +103,12 @@ def as_expr(x) -> Expr:
     raise TypeError(f"not a vector expression: {type(x).__name__}")
 
 
+def _is_number(x):
+    return type(x) in (float, complex, int) or (not isinstance(x, Expr) and isinstance(x, numbers.Number))
+
+
 def _combine(op, a, b):
-    a_s = isinstance(a, numbers.Number)
-    b_s = isinstance(b, numbers.Number)
+    a_s, b_s = _is_number(a), _is_number(b)
     if a_s and b_s:
         raise TypeError("an expression needs at least one vector")
     if b_s:
@@ -125,53 +120,62 @@ def _combine(op, a, b):
 
 def conj(x):
     """vector_arithm.hpp:495 conj(expression); the conjugate of a scalar is the scalar's."""
-    if isinstance(x, numbers.Number):
+    if _is_number(x):
         return complex(x).conjugate() if isinstance(x, complex) else x
     return Conj(as_expr(x))
+
+
+_LOAD, _CONJ = _lib.VOP["LOAD"], _lib.VOP["CONJ"]
+_BIN_OP = {op: _lib.VOP[name] for op, name in _BIN.items()}
+# (operation, scalar on the left, real scalar) -> op
+_SCA_OP = {(op, left, real): _lib.VOP[names[left] + ("R" if real else "S")]
+           for op, names in _SCA.items() for left in (False, True) for real in (False, True)}
 
 
 def compile_expr(expr: Expr):
     """Program (list of VInstr fields) and source list for pcx_vexpr_eval."""
     expr = as_expr(expr)
-    if expr.need() > _lib.VEXPR_REGS:
-        raise PcxError(_lib.ERR_UNSUPPORTED, f"expression needs {expr.need()} registers (at most 4)")
+    if expr.regs > _lib.VEXPR_REGS:
+        raise PcxError(_lib.ERR_UNSUPPORTED, f"expression needs {expr.regs} registers (at most 4)")
     srcs, index, prog = [], {}, []
 
-    def src_of(vec):
-        key = (vec.data_ptr(), vec.pack)
-        if key not in index:
-            index[key] = len(srcs)
-            srcs.append(vec)
-        return index[key]
-
-    def emit(op, d, a=0, b=0, s=0j):
-        prog.append((_lib.VOP[op], d, a, b, float(complex(s).real), float(complex(s).imag)))
-
     def gen(e, r):
-        if isinstance(e, Leaf):
-            emit("LOAD", r, src_of(e.vec))
-        elif isinstance(e, Conj):
+        kind = type(e)
+        if kind is Leaf:
+            vec = e.vec
+            key = (vec.data_ptr(), vec.pack)
+            at = index.get(key)
+            if at is None:
+                at = index[key] = len(srcs)
+                srcs.append(vec)
+            prog.append((_LOAD, r, at, 0, 0.0, 0.0))
+        elif kind is Conj:
             gen(e.expr, r)
-            emit("CONJ", r, r)
-        elif isinstance(e, Scalar):
+            prog.append((_CONJ, r, r, 0, 0.0, 0.0))
+        elif kind is Scalar:
             gen(e.expr, r)
-            right, left = _SCA[e.op]
-            name = (left if e.left else right) + ("R" if isinstance(e.scalar, numbers.Real) else "S")
-            emit(name, r, r, s=e.scalar)
+            s = e.scalar
+            real = type(s) in (float, int) or isinstance(s, numbers.Real)
+            z = complex(s)
+            prog.append((_SCA_OP[e.op, e.left, real], r, r, 0, z.real, z.imag))
+        elif e.lhs.regs >= e.rhs.regs:
+            gen(e.lhs, r)
+            gen(e.rhs, r + 1)
+            prog.append((_BIN_OP[e.op], r, r, r + 1, 0.0, 0.0))
         else:
-            if e.lhs.need() >= e.rhs.need():
-                gen(e.lhs, r)
-                gen(e.rhs, r + 1)
-                emit(_BIN[e.op], r, r, r + 1)
-            else:
-                gen(e.rhs, r)
-                gen(e.lhs, r + 1)
-                emit(_BIN[e.op], r, r + 1, r)
+            gen(e.rhs, r)
+            gen(e.lhs, r + 1)
+            prog.append((_BIN_OP[e.op], r, r + 1, r, 0.0, 0.0))
 
     gen(expr, 0)
     if len(prog) > _lib.VEXPR_MAX_PROG or len(srcs) > _lib.VEXPR_MAX_SRC:
         raise PcxError(_lib.ERR_UNSUPPORTED, "expression exceeds 64 instructions or 16 sources")
     return prog, srcs
+
+
+# the C structs, packed straight into bytes (VSource / VSource64, VInstr, VInstr64; native mode: a
+# scalar beyond FLT_MAX becomes infinite, as in ctypes)
+_PACK_SRC, _PACK_F32, _PACK_F64 = struct.Struct("@Pq").pack, struct.Struct("@iiiiff").pack, struct.Struct("@iiiidd").pack
 
 
 def _common_dtype(*vs) -> str:
@@ -184,28 +188,22 @@ def _common_dtype(*vs) -> str:
 
 def store(expr, dst, stream=None) -> None:
     """pcxo::store(expr, dst) (vector_arithm.hpp:405-447): evaluate into dst in its pack size."""
-    import ctypes as C
-
-    from .fft import _stream_ptr
-
     expr = as_expr(expr)
-    if expr.size() != dst.size():
+    if expr.n != dst.size():
         raise PcxError(_lib.ERR_SIZE_MISMATCH,
-                       f"expression size (which is {expr.size()}) differs from destination size (which is {dst.size()})")
+                       f"expression size (which is {expr.n}) differs from destination size (which is {dst.size()})")
     prog, srcs = compile_expr(expr)
     f64 = _common_dtype(dst, *srcs) == "float64"
-    VS, VI = (_lib.VSource64, _lib.VInstr64) if f64 else (_lib.VSource, _lib.VInstr)
-    S = (VS * max(1, len(srcs)))(*[VS(v.data_ptr(), v.pack) for v in srcs])
-    P = (VI * len(prog))(*[VI(*i) for i in prog])
+    pack = _PACK_F64 if f64 else _PACK_F32
+    S = b"".join([_PACK_SRC(v.data_ptr(), v.pack) for v in srcs])
+    P = b"".join([pack(*i) for i in prog])
     ev = lib().pcx_vexpr_eval_f64 if f64 else lib().pcx_vexpr_eval
-    check(ev(S, len(srcs), P, len(prog), dst.data_ptr(), dst.pack, dst.size(), _stream_ptr(stream)))
+    check(ev(S, len(srcs), P, len(prog), dst.data_ptr(), dst.pack, dst.size(), stream_ptr(stream)))
 
 
 def repack(dst, src, stream=None) -> None:
     """Pack conversion dst <- src (same size, any two pack sizes)."""
-    from .fft import _stream_ptr
-
     if src.size() != dst.size():
         raise PcxError(_lib.ERR_SIZE_MISMATCH, "repack needs equal sizes")
     rp = lib().pcx_repack_f64 if _common_dtype(dst, src) == "float64" else lib().pcx_repack
-    check(rp(dst.data_ptr(), dst.pack, src.data_ptr(), src.pack, dst.size(), _stream_ptr(stream)))
+    check(rp(dst.data_ptr(), dst.pack, src.data_ptr(), src.pack, dst.size(), stream_ptr(stream)))
