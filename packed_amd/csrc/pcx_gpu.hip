@@ -208,6 +208,10 @@ struct pcx_plan_s {
     // transform (W_N in tw_one), or k_dif
     bool    use_one      = false;
     void*   tw_one       = nullptr;
+    // natural-order 2^15 / 2^16: one pass over tiles held by one workgroup (k_tile): W_N in thread
+    // order, W_128, W_(N/128)^(c t); one workgroup per CU
+    float2* tw_tile      = nullptr;
+    int     ncu          = 0;
     // three-pass natural-order transforms of 2^21 .. 2^24 (FP64: 2^21 .. 2^23): stage tables
     // W_N2, W_Nb, W_Na and the two-level W_N1 pass table (lo, hi), in the plan's precision
     bool    use_three    = false;
@@ -335,6 +339,23 @@ extern "C" int pcx_plan_create(int64_t fft_size, int64_t sub_size, int order, pc
             if (he == hipSuccess)
                 he = gen_twiddles((float2*)p->tw_one, fft_size, 1, fft_size, st);
         }
+        if (he == hipSuccess && order == PCX_ORDER_NORMAL && lg >= kCuTileMinLog2 && lg <= kCuTileMaxLog2) {
+            const int64_t r = fft_size / kTilePoints; // tiles
+            int           dev = 0;
+            he = hipGetDevice(&dev);
+            if (he == hipSuccess)
+                he = hipDeviceGetAttribute(&p->ncu, hipDeviceAttributeMultiprocessorCount, dev);
+            if (he == hipSuccess)
+                he = hipMalloc(&p->tw_tile, sizeof(float2) * (kTilePoints + kTileEdge * (1 + r)));
+            if (he == hipSuccess) {
+                launch_tile_twiddles(p->tw_tile, lg, st);
+                he = hipGetLastError();
+            }
+            if (he == hipSuccess)
+                he = gen_twiddles(p->tw_tile + kTilePoints, kTileEdge, 1, kTileEdge, st);
+            for (int64_t t = 0; t < r && he == hipSuccess; ++t)
+                he = gen_twiddles(p->tw_tile + kTilePoints + kTileEdge * (1 + t), kTileEdge * r, t, kTileEdge, st);
+        }
         // three passes are the default: 2^21 / 2^22 / 2^23 / 2^24 in 2.74 / 2.83 / 2.93 /
         // 2.95 ms per 2 GiB forward against 3.03 / 3.67 / 4.45 / 6.00 with the four-step
         if (he == hipSuccess)
@@ -365,6 +386,7 @@ extern "C" int pcx_plan_destroy(pcx_plan_t p) {
     (void)hipFree(p->tmp);
     (void)hipFree(p->tw_dif);
     (void)hipFree(p->tw_one);
+    (void)hipFree(p->tw_tile);
     for (void* t : p->tw3)
         (void)hipFree(t);
     (void)hipFree(p->tw64_row);
@@ -556,6 +578,20 @@ struct ExtTmp {
 // 264 / 199 / 181.  FP64 2^14, four-step / one pass: 64 19.1 / 23.3, 256 48 / 32.3, 4096 790 / 484.
 constexpr int64_t kOnePassBatch = 160, kDifBatch = 48, kOnePassBatch64 = 96;
 
+// How many of a call's natural-order 2^15 / 2^16 transforms k_tile takes (one per CU and round, `ncu`
+// CUs): 2^16 in full rounds and a last one filled to more than 0.7, the others the four-step.
+// Forward in packs of 8, us, four-step / k_tile: 160 transforms 61 / 62, 180 73 / 62, 256 103 / 69,
+// 512 227 / 146, 769 331 / 244, 4096 1575 / 1120; 257 105 / 116 in two rounds, 85 in one and a
+// four-step, 300 136 / 117, 1025 460 / 313.  2^15 beyond three rounds, in one pass over halves in LDS (below) / k_tile: 257
+// 57 / 55, packs of 1 63 / 65, 513 92 / 92 and 97 / 107, 769 138 / 129 and 150 / 152, 1024 160 / 136
+// and 179 / 156, 4096 555 / 465 and 626 / 587.
+int64_t tile_batch(int lg, int64_t batch, int64_t ncu) {
+    if (lg == 15)
+        return batch > 3 * ncu ? batch : 0;
+    const int64_t last = batch % ncu;
+    return 10 * last > 7 * ncu ? batch : batch - last;
+}
+
 // src_offs / dst_offs (optional, device arrays of `batch` element offsets) replace b * dist.
 // T is the element type: float, or double for a plan made by pcx_plan_create_f64.
 template<class T>
@@ -607,6 +643,30 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
         tw_row = p->tw64_row, tw_col = p->tw64_col, twl = p->twl64, twh = p->twh64;
     else
         tw_row = p->tw_row, tw_col = p->tw_col, twl = p->twl, twh = p->twh;
+
+    // ---- one pass over a CU's registers and LDS
+    if constexpr (!F64) {
+        // offsets of multiples of 128 add under packs up to 128 and from N on
+        auto fits = [&](int lp) { return lp <= ilog2c(kTileEdge) || (lp >= p->lg && lp <= 27); };
+        if (p->tw_tile && p->auto_shape && (p->lg != kOnePassLog2 || p->use_one) && p->precision == PCX_PREC_FP32 &&
+            src_size == n && fits(src_lp) && fits(dst_lp)) {
+            if (const int64_t nb = tile_batch(p->lg, batch, p->ncu); nb > 0) {
+                TileArgs t{};
+                t.a.src = src, t.a.dst = dst, t.a.src_dist = src_dist, t.a.dst_dist = dst_dist;
+                t.a.src_size = n, t.a.nrows = nb, t.a.src_lp = src_lp, t.a.dst_lp = dst_lp;
+                t.a.conj_in = inverse, t.a.conj_out = inverse, t.a.scale = scale;
+                t.a.src_offs = src_offs, t.a.dst_offs = dst_offs;
+                t.tw = p->tw_tile, t.tw128 = p->tw_tile + kTilePoints, t.twr = t.tw128 + kTileEdge;
+                t.src_sh = src_lp < p->lg, t.dst_sh = dst_lp < p->lg;
+                launch_tile(p->lg, t, p->ncu, st);
+                HIPCHK(hipGetLastError());
+                if (nb == batch)
+                    return PCX_SUCCESS;
+                src += src_offs ? 0 : nb * src_dist, dst += dst_offs ? 0 : nb * dst_dist, batch -= nb;
+                src_offs = src_offs ? src_offs + nb : nullptr, dst_offs = dst_offs ? dst_offs + nb : nullptr;
+            }
+        }
+    }
 
     // ---- one pass: one workgroup (or several, for small sizes) per group of whole transforms
     const bool whole = p->use_one && p->precision == PCX_PREC_FP32 && batch >= (F64 ? kOnePassBatch64 : kOnePassBatch);

@@ -171,3 +171,25 @@ def test_queue_above_persistent_range(orc, pa):
     q.exec(dst.data_ptr(), src.data_ptr())
     torch.cuda.synchronize()
     _check(orc, jobs, data, dst.cpu().numpy())
+
+
+@pytest.mark.parametrize("extra", [1, 181])
+def test_queue_many_of_one_large_size(orc, pa, extra):
+    """More 2^16 transforms of each direction than the GPU has CUs, at scattered offsets: full
+    rounds of one transform per CU with a short and a nearly full last one."""
+    import torch
+
+    n, count = 1 << 16, torch.cuda.get_device_properties(0).multi_processor_count + extra
+    slots = np.random.default_rng(7).permutation(2 * count)
+    jobs = [(16, k % 2, int(slots[k]) * 2 * n, (2 * count - 1 - k) * 2 * n) for k in range(2 * count)]
+    src = torch.randn(4 * count * n, generator=torch.Generator("cuda").manual_seed(8), device="cuda")
+    dst = torch.zeros_like(src)
+    q = pa.fft_queue(jobs)
+    q.exec(dst.data_ptr(), src.data_ptr())
+    picks = [0, 1, count, 2 * count - extra - 2, 2 * count - 2, 2 * count - 1]
+    part = [jobs[k] for k in picks]
+    data = []
+    for _, _, so, _ in part:
+        x = src[so:so + 2 * n].cpu().numpy().astype(np.float64)
+        data.append(x[:n] + 1j * x[n:])
+    _check(orc, part, data, dst.cpu().numpy())

@@ -42,3 +42,39 @@ def test_shape_limits(orc, order, dtype, lg, batch):
         spec = np.empty(n, np.complex128)
         spec[slots] = src[b].to_complex()
         assert orc.rel_l2(dst[b].to_complex(), np.fft.ifft(spec)) < tol, b
+
+
+@pytest.mark.parametrize("src_pack,dst_pack", [(1, 8), (8, 1), (64, 128), (128, 0), (0, 64), (8, 256), (8, None)])
+@pytest.mark.parametrize("lg,rounds,rest", [(15, 3, 1), (16, 0, 180), (16, 1, 0), (16, 1, 1), (16, 1, 180)])
+def test_whole_transforms_per_cu(orc, lg, rounds, rest, src_pack, dst_pack):
+    """Natural-order 2^15 / 2^16 in one pass, one transform per CU and round: packs on both sides
+    (0: the whole transform, None: in place; 256 is not taken), both directions, transforms spaced
+    apart, guards between them untouched."""
+    import torch
+
+    import packed_amd as pa
+
+    n = 1 << lg
+    batch = rounds * torch.cuda.get_device_properties(0).multi_processor_count + rest
+    src_pack = src_pack or n
+    inplace, dst_pack = dst_pack is None, src_pack if dst_pack is None else dst_pack or n
+    dist = 2 * n + 64
+    src = torch.randn(batch * dist, generator=torch.Generator("cuda").manual_seed(lg + batch), device="cuda")
+    keep = src.clone()
+    tol = 2 * lg * 2.0 ** -23
+
+    def vec(t, b, pack):
+        x = t[b * dist:b * dist + 2 * n].cpu().numpy().astype(np.float64).reshape(n // pack, 2, pack)
+        return (x[:, 0] + 1j * x[:, 1]).reshape(n)
+
+    unit = pa.fft_unit(n)
+    for inverse in (False, True):
+        src.copy_(keep)
+        dst = src if inplace else torch.full((batch * dist,), 7.0, device="cuda")
+        unit.batch(dst.data_ptr(), src.data_ptr(), batch, dst_pack, dist, src_pack, dist, inverse=inverse)
+        for b in sorted({0, batch // 2, max(batch - 1 - rest, 0), batch - 1}):
+            z = vec(keep, b, src_pack)
+            want = np.fft.ifft(z) if inverse else np.fft.fft(z)
+            assert orc.rel_l2(vec(dst, b, dst_pack), want) < tol, (inverse, b)
+        gaps = dst.view(batch, dist)[:, 2 * n:]
+        assert bool((gaps == (keep.view(batch, dist)[:, 2 * n:] if inplace else 7.0)).all())
