@@ -11,7 +11,7 @@ void launch_tile(int lg, const TileArgs& a, int64_t grid, hipStream_t st) {
         hipLaunchKernelGGL(k_tile<4>, g, dim3(kTileThreads), 0, st, a);
 }
 void launch_tile_twiddles(float2* t, int lg, hipStream_t st) {
-    hipLaunchKernelGGL(k_tile_twiddles, dim3(kTilePoints / 256), dim3(256), 0, st, t, lg);
+    hipLaunchKernelGGL(k_tile_twiddles, dim3((tile_table((1 << lg) / kTilePoints) + 255) / 256), dim3(256), 0, st, t, lg);
 }
 
 } // namespace pcxd

@@ -340,21 +340,16 @@ extern "C" int pcx_plan_create(int64_t fft_size, int64_t sub_size, int order, pc
                 he = gen_twiddles((float2*)p->tw_one, fft_size, 1, fft_size, st);
         }
         if (he == hipSuccess && order == PCX_ORDER_NORMAL && lg >= kCuTileMinLog2 && lg <= kCuTileMaxLog2) {
-            const int64_t r = fft_size / kTilePoints; // tiles
-            int           dev = 0;
+            int dev = 0;
             he = hipGetDevice(&dev);
             if (he == hipSuccess)
                 he = hipDeviceGetAttribute(&p->ncu, hipDeviceAttributeMultiprocessorCount, dev);
             if (he == hipSuccess)
-                he = hipMalloc(&p->tw_tile, sizeof(float2) * (kTilePoints + kTileEdge * (1 + r)));
+                he = hipMalloc(&p->tw_tile, sizeof(float2) * tile_table((int)(fft_size / kTilePoints)));
             if (he == hipSuccess) {
                 launch_tile_twiddles(p->tw_tile, lg, st);
                 he = hipGetLastError();
             }
-            if (he == hipSuccess)
-                he = gen_twiddles(p->tw_tile + kTilePoints, kTileEdge, 1, kTileEdge, st);
-            for (int64_t t = 0; t < r && he == hipSuccess; ++t)
-                he = gen_twiddles(p->tw_tile + kTilePoints + kTileEdge * (1 + t), kTileEdge * r, t, kTileEdge, st);
         }
         // three passes are the default: 2^21 / 2^22 / 2^23 / 2^24 in 2.74 / 2.83 / 2.93 /
         // 2.95 ms per 2 GiB forward against 3.03 / 3.67 / 4.45 / 6.00 with the four-step

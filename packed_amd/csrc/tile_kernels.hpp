@@ -40,17 +40,26 @@ struct TileArgs {
     int           src_sh, dst_sh; // 1 for packs up to 128, 0 for packs >= N: poff(128 x) = 128 x << sh
 };
 
-// Table of a plan of 2^lg points: entry [slot][thread], slot = 8m + r, thread = 128 j8 + c,
-// k2 = j8 + 8m + 16r.
+// Tables of a plan of 2^lg points in one array: W_N^(c k2) at [slot][thread], slot = 8m + r,
+// thread = 128 j8 + c, k2 = j8 + 8m + 16r; then W_128; then W_(128R)^(c t) at [t][c].
+constexpr int tile_table(int r) { return kTilePoints + kTileEdge * (1 + r); }
 static __global__ __launch_bounds__(256) void k_tile_twiddles(float2* t, int lg) {
     const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (e >= kTilePoints)
+    const int r = (1 << lg) / kTilePoints, f = e - kTilePoints;
+    if (e >= tile_table(r))
         return;
-    const int     th = e & 1023, slot = e >> 10;
-    const int     k2 = (th >> 7) + 8 * (slot >> 3) + 16 * (slot & 7);
-    const int64_t x  = (int64_t)(th & 127) * k2; // below 2^14
-    double        s, c;
-    sincospi(-2.0 * (double)x / (double)((int64_t)1 << lg), &s, &c);
+    int x, n; // W_n^x
+    if (f < 0) {
+        const int th = e & 1023, slot = e >> 10;
+        x            = (th & 127) * ((th >> 7) + 8 * (slot >> 3) + 16 * (slot & 7));
+        n            = 1 << lg;
+    } else if (f < kTileEdge) {
+        x = f, n = kTileEdge;
+    } else {
+        x = (f % kTileEdge) * (f / kTileEdge - 1), n = kTileEdge * r;
+    }
+    double s, c;
+    sincospi(-2.0 * (double)x / (double)n, &s, &c);
     t[e] = float2{(float)c, (float)s};
 }
 
