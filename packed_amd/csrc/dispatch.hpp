@@ -191,10 +191,11 @@ struct FourStepT {
     int                          lg, n1, n2, g, c;
     std::array<RowLaunchT<T>, 6> rows;
     std::array<ColLaunchT<T>, 2> cols;
-    // default grid cap: workgroups that fill a CU by themselves loop over their tiles (2048);
-    // several smaller ones per CU run one tile each (0: no cap), the next workgroup's loads
-    // overlapping the others' stores (2^16 x 1024, 4096-point tiles: 429 us against 539 capped)
-    int64_t grid = 0;
+    // default grid caps of the rows and columns: workgroups that fill a CU by themselves loop over
+    // their tiles (2048); several smaller ones per CU run one tile each (0: no cap), the next
+    // workgroup's loads overlapping the others' stores (2^16 x 1024, 4096-point tiles: 429 us
+    // against 539 capped)
+    int64_t grid_row = 0, grid_col = 0;
 };
 using FourStep = FourStepT<float>;
 constexpr int64_t kWideGrid = 2048;

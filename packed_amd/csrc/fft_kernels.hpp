@@ -221,6 +221,24 @@ struct PassTw {
         }
     }
 };
+// The same with the high factor W_(2^(lg-ls))^hi from the columns' own W_A table `ta` (kPassTwA;
+// LA >= lg - ls, both tables rounded from the same values): TWN low entries alone.
+template<int LA, int TWN, class T = float>
+struct PassTwA {
+    static_assert(TwTable<LA, T>::direct, "a whole W_A table");
+    __device__ static void fill(T* t, const vec2<T>* __restrict__ twl, int tid, int nthreads) {
+        for (int e = tid; e < TWN; e += nthreads) {
+            vec2<T> w  = twl[e];
+            t[e]       = w.x;
+            t[TWN + e] = w.y;
+        }
+    }
+    __device__ static cx<T> get(const T* t, const T* ta, int lg, uint32_t e) {
+        constexpr int  LS = ilog2c(TWN);
+        const uint32_t lo = e & (TWN - 1), hi = (e >> LS) << (LA - lg + LS);
+        return cmul(cx<T>{t[lo], t[TWN + lo]}, cx<T>{ta[hi], ta[TwTable<LA, T>::NLO + hi]});
+    }
+};
 // pass-twiddle table capacity for a transform of 2^lg points (0: none needed)
 constexpr int pass_tw_entries(int lg) { return (1 << ((lg + 1) / 2)) + (1 << (lg / 2)); }
 
@@ -1034,7 +1052,10 @@ __device__ __forceinline__ void col_tile(const ColArgsT<T>& p, int64_t tile, T* 
 #pragma unroll
             for (int r = 0; r < RL; ++r) {
                 uint32_t e    = n1 * (uint32_t)out_elem<LA, false, T, PX>(jt, m, r);
-                v[m * RL + r] = cmul(v[m * RL + r], PassTw<TW, T>::get(lptw, p.twl, p.twh, p.tw_ls, p.tw_lg, e));
+                if constexpr ((PX & kPassTwA) != 0)
+                    v[m * RL + r] = cmul(v[m * RL + r], PassTwA<LA, TW, T>::get(lptw, ltw, p.tw_lg, e));
+                else
+                    v[m * RL + r] = cmul(v[m * RL + r], PassTw<TW, T>::get(lptw, p.twl, p.twh, p.tw_ls, p.tw_lg, e));
                 __builtin_amdgcn_sched_barrier(0); // one element's table reads in flight at a time
             }
     }
@@ -1092,7 +1113,9 @@ void k_col(ColArgsT<T> p) {
     T*            lre  = lds + LC::DOFF;
     T*            lim  = P::HALF ? lre : lre + DATA / 2;
     TwTable<LA, T>::fill(ltw, p.twA, threadIdx.x, NT);
-    if constexpr (TW > 0)
+    if constexpr ((PX & kPassTwA) != 0)
+        PassTwA<LA, TW, T>::fill(lptw, p.twl, threadIdx.x, NT);
+    else if constexpr (TW > 0)
         PassTw<TW, T>::fill(lptw, p.twl, p.twh, p.tw_ls, p.tw_lg, threadIdx.x, NT);
     __syncthreads();
     MfmaDft16 mf;

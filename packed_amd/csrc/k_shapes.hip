@@ -8,12 +8,20 @@ constexpr FourStep kDefault[] = {
     // and store segments in the column pass; 128 KiB of LDS, one workgroup of 1024 threads per
     // CU): 0.778 ms per 2 GiB against 0.855 ms with 64 columns; 2^15 (four-step forward, 64 rows
     // per row workgroup) 1.59 against 1.70 ms per 2 GiB
-    shape<15, 8, 7, 64, 128>(), shape<16, 9, 7, 32, 128>(), shape<17, 9, 8, 32, 64>(), shape<18, 9, 9, 32, 32>(),
+    shape<15, 8, 7, 64, 128>(), shape<16, 9, 7, 32, 128>(), shape<17, 9, 8, 32, 64>(), shape<18, 9, 9, 32, 32, kTwoTiles>(),
+    // Columns of 2^18 .. 2^20: latency of a tile's loads and stores, so two 16384-point tiles share a
+    // CU (kTwoTiles; 1024 threads each, 64 VGPRs).  One column pass forward / inverse in packs of 8,
+    // us, one tile per CU and round -> two: 2^20 x 128 683 / 653 -> 540 / 454 (4.7 TB/s), 2^19 x 256
+    // (32 columns of 32 points per thread before) 546 / 520 -> 508 / 416, 2^18 x 512 477 / 464 -> 414 /
+    // 409.  Rows stay at one group per CU: with one exchange array 2^20 x 128 forward 517 -> 480 us
+    // in packs of 8 but 460 -> 537 split, and the inverse's pass twiddles leave no room for two.
+    // Loading the next tile during a transform instead (one per CU): 656 / 534 columns, rows 540 ->
+    // 460 in packs of 8 but 528 -> 560 split.
+    // Whole calls: 2^20 x 256 2393 -> 2156 us (split 2112 -> 1952), 2^20 x 16 163 -> 157, 2^19 x 512
+    // 1867 -> 1829 (1780 -> 1702), 2^18 x 1024 1796 -> 1680 (1716 -> 1606).
     // 2^19: 512-point rows, 32 per workgroup (128-byte store segments), 1.91 against 2.03 ms per
-    // 2 GiB with 1024-point rows (an alternative); 1024-point columns 32 per tile (128-byte
-    // segments) with 32 points per thread and one LDS array: 1.83 / 1.83 ms forward / inverse
-    // against 1.85 / 1.89 with 16 per tile.  (2^20 gained nothing from the same columns.)
-    shape<19, 9, 10, 32, 32, 32 | kHalfExchange>(), shape<20, 10, 10, 16, 16>(), shape<21, 11, 10, 8, 16>(), shape<22, 12, 10, 4, 16>(),
+    // 2 GiB with 1024-point rows (an alternative).
+    shape<19, 9, 10, 32, 16, kTwoTiles>(), shape<20, 10, 10, 16, 16, kTwoTiles>(), shape<21, 11, 10, 8, 16>(), shape<22, 12, 10, 4, 16>(),
     // 2^23, 2^24: more rows per workgroup than the LDS of two workgroups per CU allows (they
     // spill, but store 4 / 2 floats per segment instead of 2 / 1): 5.03 / 5.87 ms per 2 GiB
     // forward against 7.47 / 8.94

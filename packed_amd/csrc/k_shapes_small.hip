@@ -21,6 +21,7 @@ constexpr SmallShapeT<float> kSmall[] = {
     {21, shape<19, 9, 10, 16, 8>()},  // one 34 / 32 -> 18.3 / 18.1; 2^21 40 / 39 -> 27.6 / 26.7
     {22, shape<19, 9, 10, 8, 16>()},  // 2^22 46 / 44 -> 35 / 39
     {21, shape<20, 10, 10, 8, 8>()},  // one 27.9 / 27.5 -> 23.4 / 23.1; 2^21 35 / 35 -> 33 / 31
+    {22, shape<20, 10, 10, 16, 16>()}, // up to one tile per CU: 3 39 / 41, 4 42 / 45 with the default's columns
     // the permuted orders' split at 2^20 (bit_reversed): one 25.8 / 26.7 -> 19.8 / 20.4;
     // 2^24 135 / 141 -> 111 / 117; 2^26 496 / 524 -> 485 / 484
     {26, shape<20, 12, 8, 1, 16>()},

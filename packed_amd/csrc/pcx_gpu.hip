@@ -776,9 +776,9 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
     const ThreePassT<T>* tp3 = p->use_three && p->order == PCX_ORDER_NORMAL && p->precision == PCX_PREC_FP32
                                    ? three_of<T>(p->lg)
                                    : nullptr;
-    const int64_t own_grid = tp3 || p->precision != PCX_PREC_FP32 ? kWideGrid : shape->grid;
-    const int64_t grid_col = p->grid_col >= 0 ? p->grid_col : own_grid;
-    const int64_t grid_row = p->grid_row >= 0 ? p->grid_row : own_grid;
+    const bool    wide     = tp3 || p->precision != PCX_PREC_FP32;
+    const int64_t grid_col = p->grid_col >= 0 ? p->grid_col : (wide ? kWideGrid : shape->grid_col);
+    const int64_t grid_row = p->grid_row >= 0 ? p->grid_row : (wide ? kWideGrid : shape->grid_row);
     for (int64_t b0 = 0; b0 < batch; b0 += chunk) {
         int64_t      cb = batch - b0 < chunk ? batch - b0 : chunk;
         const T*       cs  = src_offs ? src : src + b0 * src_dist;

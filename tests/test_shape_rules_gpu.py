@@ -10,7 +10,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 F32 = [(15, 47), (15, 48), (15, 159), (15, 160), (15, 161), (16, 1024), (16, 1025), (17, 128), (17, 129), (17, 513),
-       (18, 4), (18, 5), (18, 257), (19, 4), (19, 5), (19, 9), (20, 2), (20, 3), (20, 65)]
+       (18, 4), (18, 5), (18, 257), (19, 4), (19, 5), (19, 9), (20, 2), (20, 3), (20, 4), (20, 5), (20, 65)]
 F64 = [(14, 95), (14, 96), (14, 97), (15, 32), (15, 33), (15, 513), (16, 2), (16, 3), (16, 257), (17, 3), (18, 1), (18, 2),
        (19, 8), (19, 9), (20, 4), (20, 5)]
 
