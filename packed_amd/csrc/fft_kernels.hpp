@@ -142,13 +142,27 @@ __device__ __forceinline__ float buf_ld(float*, __amdgpu_buffer_rsrc_t r, uint32
 __device__ __forceinline__ double buf_ld(double*, __amdgpu_buffer_rsrc_t r, uint32_t vb, uint32_t sb) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, vb, sb, 0));
 }
+// The two adjacent parts of a pack-1 element in one access (four-byte alignment suffices).
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ cx<float> buf_ld2(float*, __amdgpu_buffer_rsrc_t r, uint32_t vb, uint32_t sb) {
+    return __builtin_bit_cast(cx<float>, __builtin_amdgcn_raw_buffer_load_b64(r, vb, sb, 0));
+}
+__device__ __forceinline__ cx<double> buf_ld2(double*, __amdgpu_buffer_rsrc_t r, uint32_t vb, uint32_t sb) {
+    return __builtin_bit_cast(cx<double>, __builtin_amdgcn_raw_buffer_load_b128(r, vb, sb, 0));
+}
+__device__ __forceinline__ void buf_st2(cx<float> v, __amdgpu_buffer_rsrc_t r, uint32_t vb, uint32_t sb) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, vb, sb, 0);
+}
+__device__ __forceinline__ void buf_st2(cx<double> v, __amdgpu_buffer_rsrc_t r, uint32_t vb, uint32_t sb) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, vb, sb, 0);
+}
 __device__ __forceinline__ void buf_st(float v, __amdgpu_buffer_rsrc_t r, uint32_t vb, uint32_t sb) {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, vb, sb, 0);
 }
 __device__ __forceinline__ void buf_st(double v, __amdgpu_buffer_rsrc_t r, uint32_t vb, uint32_t sb) {
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, vb, sb, 0);
 }
-template<class T = float>
+template<class T = float, bool ONE = false> // ONE: pack 1
 struct BufR {
     static constexpr uint32_t E = sizeof(T);
     __amdgpu_buffer_rsrc_t re, im;
@@ -158,14 +172,18 @@ struct BufR {
     __device__ BufR(const T* base, int lp, uint32_t nfl)
         : re(rsrc(base, nfl * E)), im(rsrc(base + ((int64_t)1 << lp), nfl * E)) {}
     __device__ cx<T> ld(uint32_t o, int) const {
+        if constexpr (ONE)
+            return buf_ld2((T*)nullptr, re, o * E, 0);
         return {buf_ld((T*)nullptr, re, o * E, 0), buf_ld((T*)nullptr, im, o * E, 0)};
     }
     // element at vo + so, so wave-uniform (scalar offset); the range is not checked against so
     __device__ cx<T> ld(uint32_t vo, uint32_t so, int) const {
+        if constexpr (ONE)
+            return buf_ld2((T*)nullptr, re, vo * E, so * E);
         return {buf_ld((T*)nullptr, re, vo * E, so * E), buf_ld((T*)nullptr, im, vo * E, so * E)};
     }
 };
-template<class T = float>
+template<class T = float, bool ONE = false>
 struct BufW {
     static constexpr uint32_t E = sizeof(T);
     __amdgpu_buffer_rsrc_t re, im;
@@ -175,18 +193,22 @@ struct BufW {
     __device__ BufW(T* base, int lp, uint32_t nfl)
         : re(rsrc(base, nfl * E)), im(rsrc(base + ((int64_t)1 << lp), nfl * E)) {}
     __device__ void st(uint32_t o, cx<T> v, int) const {
+        if constexpr (ONE)
+            return buf_st2(v, re, o * E, 0);
         buf_st(v.x, re, o * E, 0);
         buf_st(v.y, im, o * E, 0);
     }
     __device__ void st(uint32_t vo, uint32_t so, cx<T> v, int) const {
+        if constexpr (ONE)
+            return buf_st2(v, re, vo * E, so * E);
         buf_st(v.x, re, vo * E, so * E);
         buf_st(v.y, im, vo * E, so * E);
     }
 };
-template<bool UNI, class T = float>
-using RdView = typename std::conditional<UNI, BufR<T>, CxPtr<T>>::type;
-template<bool UNI, class T = float>
-using WrView = typename std::conditional<UNI, BufW<T>, CxPtrW<T>>::type;
+template<bool UNI, class T = float, bool ONE = false>
+using RdView = typename std::conditional<UNI, BufR<T, ONE>, CxPtr<T>>::type;
+template<bool UNI, class T = float, bool ONE = false>
+using WrView = typename std::conditional<UNI, BufW<T, ONE>, CxPtrW<T>>::type;
 
 // LDS copy of the two-level W_N table for four-step pass twiddles, TWN complex entries
 // (lo + hi, TWN >= 4); TWN == 2 reads both levels from global memory instead.
@@ -326,6 +348,8 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
     constexpr int STR = S::STRIDE;
     constexpr int R0  = P::first_radix;
     constexpr int RL  = P::last_radix;
+    constexpr bool ONE = (PX & kPack1) != 0;
+    const int      slp = ONE ? 0 : p.src_lp, dlp = ONE ? 0 : p.dst_lp;
 
     const int      t      = threadIdx.x;
     const int      g      = t / TA;
@@ -397,17 +421,17 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
     // ------------------------------------------------------------------ load
     bool loaded = false;
     if constexpr ((LD == LD_CONTIG && TILE) || (LD == LD_PERM && TILEP)) {
-        const int64_t sd = tile_dist(p.src_lp, p.src_dist);
+        const int64_t sd = tile_dist(slp, p.src_dist);
         if (tile_ok(p.src_offs, sd)) {
             const uint32_t dist = (uint32_t)sd;
-            const BufR<T>  src(p.src + row0 * p.src_dist, p.src_lp, tile_range(p.src_lp, dist));
+            const BufR<T>  src(p.src + row0 * p.src_dist, slp, tile_range(slp, dist));
             const bool     ez = (int64_t)te < p.src_size; // zero extension past src_size
             // a permuted row holds frequency slot_freq(e) at position e
             const int      f  = LD == LD_PERM ? (int)slot_freq(ORD, (uint32_t)te, LA) : te;
 #pragma unroll
             for (int u = 0; u < PPT; ++u) {
                 const int gg = tg + u * TROWS;
-                cx<T>     x  = src.ld((uint32_t)gg * dist + poff((uint32_t)te, p.src_lp), p.nt_load);
+                cx<T>     x  = src.ld((uint32_t)gg * dist + poff((uint32_t)te, slp), p.nt_load);
                 x            = ez ? x : cx<T>{T(0), T(0)};
                 const int o  = gg * STR + f + (f >> 5);
                 lre[o]       = x.x;
@@ -426,17 +450,17 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
     }
     if (loaded) {
     } else if constexpr (LD == LD_CONTIG) {
-        const RdView<UNI, T> src(tbase(p.src, p.src_offs, p.src_dist, btu), p.src_lp);
+        const RdView<UNI, T, ONE> src(tbase(p.src, p.src_offs, p.src_dist, btu), slp);
         if (row_ok && (int64_t)(k2l + 1) << LA <= p.src_size) { // whole row inside the source
             if constexpr (P::HALF) {
                 // one per-lane offset plus scalar offsets: the 2^14-point plans need the registers
-                const uint32_t vo = poff((uint32_t)jt, p.src_lp);
+                const uint32_t vo = poff((uint32_t)jt, slp);
 #pragma unroll
                 for (int m = 0; m < PPT / R0; ++m)
 #pragma unroll
                     for (int r = 0; r < R0; ++r) {
                         uint32_t c    = (uint32_t)(in_elem<LA, false, T, PX>(jt, m, r) - jt) + (k2l << LA);
-                        v[m * R0 + r] = src.ld(vo, poff(c, p.src_lp), p.nt_load);
+                        v[m * R0 + r] = src.ld(vo, poff(c, slp), p.nt_load);
                     }
             } else {
 #pragma unroll
@@ -444,7 +468,7 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
 #pragma unroll
                     for (int r = 0; r < R0; ++r) {
                         uint32_t i    = (uint32_t)in_elem<LA, false, T, PX>(jt, m, r) + (k2l << LA);
-                        v[m * R0 + r] = src.ld(poff(i, p.src_lp), p.nt_load);
+                        v[m * R0 + r] = src.ld(poff(i, slp), p.nt_load);
                     }
             }
         } else {
@@ -454,7 +478,7 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
                 for (int r = 0; r < R0; ++r) {
                     uint32_t i    = (uint32_t)in_elem<LA, false, T, PX>(jt, m, r) + (k2l << LA);
                     bool     ok   = row_ok && i < p.src_size;
-                    cx<T>    x    = src.ld(ok ? poff(i, p.src_lp) : 0u, p.nt_load);
+                    cx<T>    x    = src.ld(ok ? poff(i, slp) : 0u, p.nt_load);
                     v[m * R0 + r] = ok ? x : cx<T>{T(0), T(0)};
                 }
         }
@@ -474,21 +498,21 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
             }
         };
         if constexpr (LD == LD_PERM) {
-            const RdView<UNI, T> src(tbase(p.src, p.src_offs, p.src_dist, btu), p.src_lp);
+            const RdView<UNI, T, ONE> src(tbase(p.src, p.src_offs, p.src_dist, btu), slp);
             uint32_t          base = brev_bits(k2, p.rows_lg) << LA;
 #pragma unroll
             for (int u = 0; u < PPT; ++u) {
-                cx<T> x = src.ld(row_ok ? poff(base + jt + u * TA, p.src_lp) : 0u, p.nt_load);
+                cx<T> x = src.ld(row_ok ? poff(base + jt + u * TA, slp) : 0u, p.nt_load);
                 v[u] = row_ok ? x : cx<T>{T(0), T(0)};
             }
         } else {
-            const RdView<UNI, T> src(tbase(p.src, p.src_offs, p.src_dist, row0 >> p.rows_lg), p.src_lp);
+            const RdView<UNI, T, ONE> src(tbase(p.src, p.src_offs, p.src_dist, row0 >> p.rows_lg), slp);
 #pragma unroll
             for (int u = 0; u < PPT; ++u) {
                 int     idx = t + u * NT;
                 int64_t rw  = row0 + idx % G;
                 bool    ok  = rw < p.nrows;
-                cx<T>   x   = src.ld(ok ? poff((uint32_t)(rw & rmask) + ((uint32_t)(idx / G) << p.rows_lg), p.src_lp)
+                cx<T>   x   = src.ld(ok ? poff((uint32_t)(rw & rmask) + ((uint32_t)(idx / G) << p.rows_lg), slp)
                                         : 0u,
                                      p.nt_load);
                 v[u]        = ok ? x : cx<T>{T(0), T(0)};
@@ -518,11 +542,11 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
             // element slot_freq(order, s).  All loads first, then the LDS writes: interleaving
             // them let the compiler wait for each load before the next one (2^11: 1.27 ms per
             // 2 GiB against 0.76 for the forward transform).
-            const RdView<UNI, T> src(tbase(p.src, p.src_offs, p.src_dist, btu), p.src_lp);
+            const RdView<UNI, T, ONE> src(tbase(p.src, p.src_offs, p.src_dist, btu), slp);
             uint32_t          base = brev_bits(k2, p.rows_lg) << LA;
 #pragma unroll
             for (int u = 0; u < PPT; ++u) {
-                cx<T> x = src.ld(row_ok ? poff(base + jt + u * TA, p.src_lp) : 0u, p.nt_load);
+                cx<T> x = src.ld(row_ok ? poff(base + jt + u * TA, slp) : 0u, p.nt_load);
                 v[u]    = row_ok ? x : cx<T>{T(0), T(0)};
             }
 #pragma unroll
@@ -539,7 +563,7 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
             // LD_STRIDED, row-fastest: element k1 of row k2 sits at slot k2 + (k1 << rows_lg); the
             // stage-0 inputs of this thread's butterflies go straight to registers, G consecutive
             // slots per wave and element (the rows of a workgroup lie in one transform)
-            const RdView<UNI, T> src(tbase(p.src, p.src_offs, p.src_dist, row0 >> p.rows_lg), p.src_lp);
+            const RdView<UNI, T, ONE> src(tbase(p.src, p.src_offs, p.src_dist, row0 >> p.rows_lg), slp);
             const int64_t        rw = row0 + ga;
             const bool           ok = rw < p.nrows;
             const uint32_t       kb = (uint32_t)(rw & rmask);
@@ -548,12 +572,12 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
 #pragma unroll
                 for (int r = 0; r < R0; ++r) {
                     const uint32_t k1 = (uint32_t)in_elem<LA, false, T, PX>(ja, m, r);
-                    cx<T>          x  = src.ld(ok ? poff(kb + (k1 << p.rows_lg), p.src_lp) : 0u, p.nt_load);
+                    cx<T>          x  = src.ld(ok ? poff(kb + (k1 << p.rows_lg), slp) : 0u, p.nt_load);
                     v[m * R0 + r]     = ok ? x : cx<T>{T(0), T(0)};
                 }
         } else { // LD_STRIDED: element k1 of row k2 sits at slot k2 + (k1 << rows_lg)
             // (the rows of a workgroup lie in one transform: G divides the rows per transform)
-            const RdView<UNI, T> src(tbase(p.src, p.src_offs, p.src_dist, row0 >> p.rows_lg), p.src_lp);
+            const RdView<UNI, T, ONE> src(tbase(p.src, p.src_offs, p.src_dist, row0 >> p.rows_lg), slp);
 #pragma unroll
             for (int u = 0; u < PPT; ++u) {
                 int     idx = t + u * NT;
@@ -561,7 +585,7 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
                 int     k1  = idx / G;
                 int64_t rw  = row0 + gg;
                 bool    ok  = rw < p.nrows;
-                cx<T>   x   = src.ld(ok ? poff((uint32_t)(rw & rmask) + ((uint32_t)k1 << p.rows_lg), p.src_lp) : 0u,
+                cx<T>   x   = src.ld(ok ? poff((uint32_t)(rw & rmask) + ((uint32_t)k1 << p.rows_lg), slp) : 0u,
                                      p.nt_load);
                 x           = ok ? x : cx<T>{T(0), T(0)};
                 int o  = gg * STR + k1 + (k1 >> 5);
@@ -626,7 +650,7 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
     // ------------------------------------------------------------------ store
     bool stored = false;
     if constexpr ((ST == ST_CONTIG && TILE) || (ST == ST_PERM && TILEP)) {
-        const int64_t dd = tile_dist(p.dst_lp, p.dst_dist);
+        const int64_t dd = tile_dist(dlp, p.dst_dist);
         if (tile_ok(p.dst_offs, dd)) {
             __syncthreads(); // the last stage's LDS reads are done
 #pragma unroll
@@ -639,13 +663,13 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
                 }
             __syncthreads();
             const uint32_t dist = (uint32_t)dd;
-            const BufW<T>  dst(p.dst + row0 * p.dst_dist, p.dst_lp, tile_range(p.dst_lp, dist));
+            const BufW<T>  dst(p.dst + row0 * p.dst_dist, dlp, tile_range(dlp, dist));
             const int      f = ST == ST_PERM ? (int)slot_freq(ORD, (uint32_t)opaque_after_memory(te), LA) : te;
 #pragma unroll
             for (int u = 0; u < PPT; ++u) {
                 const int gg = tg + u * TROWS;
                 const int o  = gg * STR + f + (f >> 5);
-                dst.st((uint32_t)gg * dist + poff((uint32_t)te, p.dst_lp), cx<T>{lre[o], lim[o]}, p.nt_store);
+                dst.st((uint32_t)gg * dist + poff((uint32_t)te, dlp), cx<T>{lre[o], lim[o]}, p.nt_store);
             }
             stored = true;
         }
@@ -653,15 +677,15 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
     if (stored) {
     } else if constexpr (ST == ST_CONTIG) {
         if (row_ok) {
-            const WrView<UNI, T> dst(tbase(p.dst, p.dst_offs, p.dst_dist, btu), p.dst_lp);
+            const WrView<UNI, T, ONE> dst(tbase(p.dst, p.dst_offs, p.dst_dist, btu), dlp);
             if constexpr (P::HALF) {
-                const uint32_t vo = poff((uint32_t)jt, p.dst_lp);
+                const uint32_t vo = poff((uint32_t)jt, dlp);
 #pragma unroll
                 for (int m = 0; m < PPT / RL; ++m)
 #pragma unroll
                     for (int r = 0; r < RL; ++r) {
                         uint32_t c = (uint32_t)(out_elem<LA, false, T, PX>(jt, m, r) - jt) + (k2 << LA);
-                        dst.st(vo, poff(c, p.dst_lp), v[m * RL + r], p.nt_store);
+                        dst.st(vo, poff(c, dlp), v[m * RL + r], p.nt_store);
                     }
             } else {
 #pragma unroll
@@ -669,7 +693,7 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
 #pragma unroll
                     for (int r = 0; r < RL; ++r) {
                         uint32_t i = (uint32_t)out_elem<LA, false, T, PX>(jt, m, r) + (k2 << LA);
-                        dst.st(poff(i, p.dst_lp), v[m * RL + r], p.nt_store);
+                        dst.st(poff(i, dlp), v[m * RL + r], p.nt_store);
                     }
             }
         }
@@ -710,27 +734,27 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
             v[u].y = lre[pos(u)];
         if constexpr (ST == ST_PERM) {
             if (row_ok) {
-                const WrView<UNI, T> dst(tbase(p.dst, p.dst_offs, p.dst_dist, btu), p.dst_lp);
+                const WrView<UNI, T, ONE> dst(tbase(p.dst, p.dst_offs, p.dst_dist, btu), dlp);
                 uint32_t          base = brev_bits(k2, p.rows_lg) << LA;
 #pragma unroll
                 for (int u = 0; u < PPT; ++u)
-                    dst.st(poff(base + jt + u * TA, p.dst_lp), v[u], p.nt_store);
+                    dst.st(poff(base + jt + u * TA, dlp), v[u], p.nt_store);
             }
         } else {
-            const WrView<UNI, T> dst(tbase(p.dst, p.dst_offs, p.dst_dist, row0 >> p.rows_lg), p.dst_lp);
+            const WrView<UNI, T, ONE> dst(tbase(p.dst, p.dst_offs, p.dst_dist, row0 >> p.rows_lg), dlp);
 #pragma unroll
             for (int u = 0; u < PPT; ++u) {
                 int     idx = t + u * NT;
                 int64_t rw  = row0 + idx % G;
                 if (rw < p.nrows)
-                    dst.st(poff((uint32_t)(rw & rmask) + ((uint32_t)(idx / G) << p.rows_lg), p.dst_lp), v[u],
+                    dst.st(poff((uint32_t)(rw & rmask) + ((uint32_t)(idx / G) << p.rows_lg), dlp), v[u],
                            p.nt_store);
             }
         }
     } else if constexpr (ALT_ST) {
         // ST_STRIDED, row-fastest: element k1 of row k2 goes to slot k2 + (k1 << rows_lg), G
         // consecutive slots per wave and element, straight from registers
-        const WrView<UNI, T> dst(tbase(p.dst, p.dst_offs, p.dst_dist, row0 >> p.rows_lg), p.dst_lp);
+        const WrView<UNI, T, ONE> dst(tbase(p.dst, p.dst_offs, p.dst_dist, row0 >> p.rows_lg), dlp);
         const int64_t        rw = row0 + ga;
         if (rw < p.nrows) {
 #pragma unroll
@@ -738,7 +762,7 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
 #pragma unroll
                 for (int r = 0; r < RL; ++r) {
                     const uint32_t k1 = (uint32_t)out_elem<LA, false, T, PX>(ja, m, r);
-                    dst.st(poff(ko2 + (k1 << p.rows_lg), p.dst_lp), v[m * RL + r], p.nt_store);
+                    dst.st(poff(ko2 + (k1 << p.rows_lg), dlp), v[m * RL + r], p.nt_store);
                 }
         }
     } else {
@@ -754,7 +778,7 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
         __syncthreads();
         if constexpr (ST == ST_PERM) {
             if (row_ok) {
-                const WrView<UNI, T> dst(tbase(p.dst, p.dst_offs, p.dst_dist, btu), p.dst_lp);
+                const WrView<UNI, T, ONE> dst(tbase(p.dst, p.dst_offs, p.dst_dist, btu), dlp);
                 uint32_t          base = brev_bits(k2, p.rows_lg) << LA;
 #pragma unroll
                 for (int u = 0; u < PPT; ++u) {
@@ -764,11 +788,11 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
                         o = paddr(perm_base<LA, ORD, T, PX>(jt), brevc(u, ilog2c(PPT)));
                     else
                         o = paddr(perm_elem<LA, ORD, T, PX>(jt, u), 0);
-                    dst.st(poff(base + s, p.dst_lp), cx<T>{lre[o], lim[o]}, p.nt_store);
+                    dst.st(poff(base + s, dlp), cx<T>{lre[o], lim[o]}, p.nt_store);
                 }
             }
         } else { // ST_STRIDED: element k1 of row k2 goes to slot k2 + (k1 << rows_lg)
-            const WrView<UNI, T> dst(tbase(p.dst, p.dst_offs, p.dst_dist, row0 >> p.rows_lg), p.dst_lp);
+            const WrView<UNI, T, ONE> dst(tbase(p.dst, p.dst_offs, p.dst_dist, row0 >> p.rows_lg), dlp);
 #pragma unroll
             for (int u = 0; u < PPT; ++u) {
                 int     idx = t + u * NT;
@@ -777,7 +801,7 @@ __device__ __forceinline__ void row_group(const RowArgsT<T>& p, int64_t wg, T* l
                 int64_t rw  = row0 + gg;
                 if (rw < p.nrows) {
                     int o = gg * STR + k1 + (k1 >> 5);
-                    dst.st(poff((uint32_t)(rw & rmask) + ((uint32_t)k1 << p.rows_lg), p.dst_lp), cx<T>{lre[o], lim[o]},
+                    dst.st(poff((uint32_t)(rw & rmask) + ((uint32_t)k1 << p.rows_lg), dlp), cx<T>{lre[o], lim[o]},
                            p.nt_store);
                 }
             }

@@ -5,10 +5,9 @@ namespace pcxd {
 
 void launch_tile(int lg, const TileArgs& a, int64_t grid, hipStream_t st) {
     const dim3 g((unsigned)std::min<int64_t>(a.a.nrows, grid));
-    if (lg == 15)
-        hipLaunchKernelGGL(k_tile<2>, g, dim3(kTileThreads), 0, st, a);
-    else
-        hipLaunchKernelGGL(k_tile<4>, g, dim3(kTileThreads), 0, st, a);
+    const bool one = a.a.src_lp == 0 && a.a.dst_lp == 0;
+    const auto f   = lg == 15 ? (one ? k_tile<2, true> : k_tile<2, false>) : (one ? k_tile<4, true> : k_tile<4, false>);
+    hipLaunchKernelGGL(f, g, dim3(kTileThreads), 0, st, a);
 }
 void launch_tile_twiddles(float2* t, int lg, hipStream_t st) {
     hipLaunchKernelGGL(k_tile_twiddles, dim3((tile_table((1 << lg) / kTilePoints) + 255) / 256), dim3(256), 0, st, t, lg);

@@ -27,8 +27,9 @@ namespace pcxk {
 // Plan options PX: a points-per-thread override in the low byte (the latency-bound fused
 // kernels run 2^14 with 16), kHalfExchange to take the one-array exchange (Plan::HALF) below
 // the size where it is the default, kTwChain (below), and kPassTwA: the pass twiddles of k_col take
-// their high factor from the W_A table (PassTwA).
-constexpr int kHalfExchange = 0x200, kPassTwA = 0x1000;
+// their high factor from the W_A table (PassTwA).  kPack1: k_row's source and destination have pack
+// 1, each element's two parts move in one access.
+constexpr int kHalfExchange = 0x200, kPassTwA = 0x1000, kPack1 = 0x2000;
 // kTwChain: stage twiddle exponents by one addition per twiddle (TwTable::Seq) instead of one
 // multiply each.  For kernels that run one transform per workgroup (no loop to hoist the
 // per-thread twiddle addresses out of, and no registers to keep them in).

@@ -24,7 +24,7 @@
 // W_N^((128T+c) k2), 512 KiB at R = 4, applied per tile, did not stay in L2 beside the stream: 760
 // against 556 us for 2048 transforms of 2^16 with and without its loads.)
 // 2 GiB of 2^16 split 1560 (two passes) -> 990 us, 4.3 TB/s; in packs of 8 1575 -> 1120, of 1 1880 ->
-// 1330; 2^15 (one pass over LDS halves) 1020 -> 900.
+// 1330 with 4-byte accesses (2^25 points 177, 149 with both parts of an element in one); 2^15 (one pass over LDS halves) 1020 -> 900.
 #pragma once
 #include "fft_kernels.hpp"
 
@@ -127,12 +127,14 @@ __device__ __forceinline__ void tile_fft128(cf* v, int j8, const float2* tw128, 
     }
 }
 
-template<int R>
+// ONE: pack 1 on both sides
+template<int R, bool ONE>
 __global__ __launch_bounds__(kTileThreads, 4) void k_tile(TileArgs q) {
     constexpr int E = kTileEdge, RS = kTileRowStride, V = 16;
     static_assert(R == 2 || R == 4, "two or four tiles");
     __shared__ float lds[tile_lds_floats<R>()];
     const RowArgs&   p   = q.a;
+    const int        slp = ONE ? 0 : p.src_lp, dlp = ONE ? 0 : p.dst_lp;
     const int        tid = threadIdx.x;
     auto             ln  = [&] { return opaque(tid) & (E - 1); };          // column c, or row k2
     const int        jb  = __builtin_amdgcn_readfirstlane(tid >> 7);       // butterfly index j8
@@ -148,13 +150,16 @@ __global__ __launch_bounds__(kTileThreads, 4) void k_tile(TileArgs q) {
     // (addresses are made opaque per use: loop-invariant, they would all be hoisted and spilled)
     auto load = [&](cf* v, const TileBuf& src, int T) {
         const int      sh = opaque_s(q.src_sh);
-        const uint32_t vi = lane_at(p.src_lp);
-        const uint32_t im = 4u << p.src_lp;
+        const uint32_t vi = lane_at(slp);
+        const uint32_t im = 4u << slp;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int r = 0; r < V; ++r) { // element j8 + 8r
             const uint32_t o = (uint32_t)(4 * (E * T + E * R * 8 * r)) << sh;
-            v[r]             = cf{buf_ld((float*)nullptr, src.r, vi, o), buf_ld((float*)nullptr, src.r, vi, o + im)};
+            if constexpr (ONE)
+                v[r] = buf_ld2((float*)nullptr, src.r, vi, o);
+            else
+                v[r] = cf{buf_ld((float*)nullptr, src.r, vi, o), buf_ld((float*)nullptr, src.r, vi, o + im)};
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -292,13 +297,18 @@ __global__ __launch_bounds__(kTileThreads, 4) void k_tile(TileArgs q) {
         tile_pin<V>(v);
         tile_fft128(v, jb, q.tw128, [&](cf* u) { x(u, std::false_type{}); });
         const int      sh = opaque_s(q.dst_sh);
-        const uint32_t vo = lane_at(p.dst_lp);
-        const uint32_t im = 4u << p.dst_lp;
+        const uint32_t vo = lane_at(dlp);
+        const uint32_t im = 4u << dlp;
 #pragma unroll
         for (int s = 0; s < V; ++s) {
             const uint32_t o = (uint32_t)(4 * (E * t + E * R * el(s))) << sh;
-            buf_st(v[s].x * p.scale, dst.r, vo, o);
-            buf_st(v[s].y * so_, dst.r, vo, o + im);
+            const cf       y{v[s].x * p.scale, v[s].y * so_};
+            if constexpr (ONE) {
+                buf_st2(y, dst.r, vo, o);
+            } else {
+                buf_st(y.x, dst.r, vo, o);
+                buf_st(y.y, dst.r, vo, o + im);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
     };
