@@ -43,7 +43,7 @@ const std::array<std::array<RowLaunchT<double>, 5>, kMaxSinglePass64> kSingle64 
     single_table64(std::make_integer_sequence<int, kMaxSinglePass64>{});
 
 // 2^14 doubles in one pass: 16 points per thread, 1024 threads, 132 KiB of LDS (one array).
-const std::array<RowLaunchT<double>, 5> kOnePass64 = single_set64<kOnePassLog2_64, 16>();
+const std::array<RowLaunchT<double>, 5> kOnePass64 = single_set64<kOnePassLog2_64, 16 | kNoRot>();
 
 // Three-pass natural-order transforms of 2^21 .. 2^23 doubles: tiles of 8192 points (128 KiB),
 // first-pass columns of 2^7 / 2^8 (64 / 32 per tile, 512- / 256-byte segments), 64 second-pass

@@ -13,10 +13,10 @@ namespace {
 // 2^14 17.7 / 60.7 / 793 -> 12.5 / 52.8 / 729.
 template<int LA>
 constexpr int single_px() {
-    return LA == 14 ? 16 : (LA == 13 ? 16 | kHalfExchange : 0);
+    return LA == 14 ? 16 | kNoRot : (LA == 13 ? 16 | kHalfExchange | kNoRot : 0);
 }
 // 2^15 points in one pass: 32 points per thread, 1024 threads, 132 KiB of LDS (one array).
-constexpr int kOnePassPx = 32 | kTwChain;
+constexpr int kOnePassPx = 32 | kTwChain | kNoRot;
 
 template<int LA, int PX = single_px<LA>()>
 constexpr RowSet single_set() {
