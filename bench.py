@@ -65,8 +65,17 @@ def profile_figure(name: str, key: str):
 def measured_traffic(log2n: int, batch: int, dtype: str = "float32"):
     """HBM bytes per step from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary of this
     workload (counters scaled by a plain copy of the same bytes); None for other shapes."""
-    tag = "" if dtype == "float32" else "f64_"
-    return profile_figure(f"fft_fourstep_{tag}n{1 << log2n}_b{batch}_hbm_traffic.md", "traffic_bytes_per_step")
+    return profile_figure(traffic_profile(log2n, batch, dtype), "traffic_bytes_per_step")
+
+
+def one_pass(log2n: int, dtype: str) -> bool:
+    """Sizes whose full batches run with one transform per CU (k_tile)."""
+    return dtype == "float32" and log2n in (15, 16)
+
+
+def traffic_profile(log2n: int, batch: int, dtype: str) -> str:
+    form = "tile_" if one_pass(log2n, dtype) else "fourstep_" + ("" if dtype == "float32" else "f64_")
+    return f"fft_{form}n{1 << log2n}_b{batch}_hbm_traffic.md"
 
 
 def time_steps(fn, steps, warmup):
@@ -282,10 +291,12 @@ def main():
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic,
-            "traffic_source": (f"profiles/fft_fourstep_{'f64_' if f64 else ''}n{n}_b{batch}_hbm_traffic.md: "
+            "traffic_source": (f"profiles/{traffic_profile(args.log2n, batch, args.dtype)}: "
                                "rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE of this workload, scaled by a plain copy"
                                if traffic else None),
-            "kernel": "four-step column pass k_col + row pass k_row (one step = one launch of each)",
+            "kernel": ("k_tile, one transform per CU (one step = one launch)"
+                       if args.precision == "fp32" and one_pass(args.log2n, args.dtype)
+                       else "four-step column pass k_col + row pass k_row (one step = one launch of each)"),
         },
         "inverse": {"ms": round(ms_inv, 4), "gflops": round(flops / (ms_inv * 1e-3) / 1e9, 1)},
         "bit_reversed": {"ms": round(ms_br, 4), "gflops": round(flops / (ms_br * 1e-3) / 1e9, 1),

@@ -21,7 +21,8 @@ constexpr FourStep kDefault[] = {
     // 1867 -> 1829 (1780 -> 1702), 2^18 x 1024 1796 -> 1680 (1716 -> 1606).
     // 2^19: 512-point rows, 32 per workgroup (128-byte store segments), 1.91 against 2.03 ms per
     // 2 GiB with 1024-point rows (an alternative).
-    shape<19, 9, 10, 32, 16, kTwoTiles>(), shape<20, 10, 10, 16, 16, kTwoTiles>(), shape<21, 11, 10, 8, 16>(), shape<22, 12, 10, 4, 16>(),
+    shape<19, 9, 10, 32, 16, kTwoTiles>(), shape<20, 10, 10, 16, 16, kTwoTiles>(),
+    shape<21, 11, 10, 8, 16>(), shape<22, 12, 10, 4, 16>(),
     // 2^23, 2^24: more rows per workgroup than the LDS of two workgroups per CU allows (they
     // spill, but store 4 / 2 floats per segment instead of 2 / 1): 5.03 / 5.87 ms per 2 GiB
     // forward against 7.47 / 8.94

@@ -24,7 +24,8 @@
 // W_N^((128T+c) k2), 512 KiB at R = 4, applied per tile, did not stay in L2 beside the stream: 760
 // against 556 us for 2048 transforms of 2^16 with and without its loads.)
 // 2 GiB of 2^16 split 1560 (two passes) -> 990 us, 4.3 TB/s; in packs of 8 1575 -> 1120, of 1 1880 ->
-// 1330 with 4-byte accesses (2^25 points 177, 149 with both parts of an element in one); 2^15 (one pass over LDS halves) 1020 -> 900.
+// 1330 with 4-byte accesses (2^25 points 177, 149 with both parts of an element in one); 2^15 (one
+// pass over LDS halves) 1020 -> 900.
 #pragma once
 #include "fft_kernels.hpp"
 
