@@ -1526,6 +1526,26 @@ int queue_run_group(pcx_queue_t q, const QGroup& g, float* dst, const float* src
                      q->dst_offs + g.first, &ext);
 }
 
+// Runs fn, which enqueues work on st through the queue's intermediate, after the intermediate's last
+// use on any stream.  (In a capture there is nothing to order: the replay is ordered when it is launched.)
+template<class F>
+int queue_on_tmp(pcx_queue_t q, hipStream_t st, F&& fn) {
+    if (!q->tmp)
+        return fn();
+    std::lock_guard<std::mutex> lock(q->mu);
+    hipStreamCaptureStatus      cs = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(st, &cs));
+    const bool capturing = cs != hipStreamCaptureStatusNone;
+    if (q->tmp_used && q->tmp_stream != st && !capturing)
+        HIPCHK(hipStreamWaitEvent(st, q->tmp_ev, 0));
+    const int e = fn();
+    if (!capturing) { // also after an error: what was enqueued before it uses the intermediate
+        HIPCHK(hipEventRecord(q->tmp_ev, st));
+        q->tmp_stream = st, q->tmp_used = true;
+    }
+    return e;
+}
+
 int queue_run(pcx_queue_t q, float* dst, const float* src, hipStream_t st) {
     if (q->nitems > 0) {
         QueueArgs a{};
@@ -1536,26 +1556,12 @@ int queue_run(pcx_queue_t q, float* dst, const float* src, hipStream_t st) {
         launch_queue(a, std::min<int>(q->grid, q->nitems), st);
         HIPCHK(hipGetLastError());
     }
-    if (!q->tmp) {
+    return queue_on_tmp(q, st, [&] {
         for (const auto& g : q->groups)
             if (int e = queue_run_group(q, g, dst, src, st))
                 return e;
-        return PCX_SUCCESS;
-    }
-    std::lock_guard<std::mutex> lock(q->mu);
-    hipStreamCaptureStatus      cs = hipStreamCaptureStatusNone;
-    HIPCHK(hipStreamIsCapturing(st, &cs));
-    const bool capturing = cs != hipStreamCaptureStatusNone;
-    if (q->tmp_used && q->tmp_stream != st && !capturing)
-        HIPCHK(hipStreamWaitEvent(st, q->tmp_ev, 0));
-    for (const auto& g : q->groups)
-        if (int e = queue_run_group(q, g, dst, src, st))
-            return e;
-    if (!capturing) {
-        HIPCHK(hipEventRecord(q->tmp_ev, st));
-        q->tmp_stream = st, q->tmp_used = true;
-    }
-    return PCX_SUCCESS;
+        return (int)PCX_SUCCESS;
+    });
 }
 
 // Frees the device side of the item list and the groups (the job list and settings stay).
@@ -1759,8 +1765,11 @@ extern "C" int pcx_queue_capture(pcx_queue_t q, float* dst, const float* src, vo
 extern "C" int pcx_queue_launch(pcx_queue_t q, void* stream) {
     if (!q || !q->exec)
         return fail(PCX_ERR_INVALID_ARGUMENT, "queue has no captured graph");
-    HIPCHK(hipGraphLaunch(q->exec, (hipStream_t)stream));
-    return PCX_SUCCESS;
+    // the graph's kernels use the same intermediate as the eager calls
+    return queue_on_tmp(q, (hipStream_t)stream, [&] {
+        HIPCHK(hipGraphLaunch(q->exec, (hipStream_t)stream));
+        return (int)PCX_SUCCESS;
+    });
 }
 
 extern "C" int pcx_queue_work(pcx_queue_t q, double* flops, double* bytes) {

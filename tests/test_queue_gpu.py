@@ -193,3 +193,47 @@ def test_queue_many_of_one_large_size(orc, pa, extra):
         x = src[so:so + 2 * n].cpu().numpy().astype(np.float64)
         data.append(x[:n] + 1j * x[n:])
     _check(orc, part, data, dst.cpu().numpy())
+
+
+@pytest.mark.parametrize("graph_first", [False, True])
+def test_replay_and_eager_pass_on_two_streams(orc, pa, graph_first):
+    """An eager pass on one stream and a replay of the captured graph on another, with no
+    synchronisation between them: both go through the queue's one intermediate, so the later waits."""
+    import torch
+
+    jobs, at = [], 0
+    for lg, count in ((17, 24), (18, 12), (20, 5)):
+        for k in range(count):
+            jobs.append((lg, k % 2, at, at))
+            at += 2 << lg
+    gen = torch.Generator("cuda").manual_seed(9)
+    srcs = [torch.randn(at, generator=gen, device="cuda") for _ in range(2)]
+    dsts = [torch.zeros_like(s) for s in srcs]
+    q = pa.fft_queue(jobs)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    q.capture(dsts[1].data_ptr(), srcs[1].data_ptr(), streams[1])
+    torch.cuda.synchronize()
+
+    def eager():
+        q.exec(dsts[0].data_ptr(), srcs[0].data_ptr(), streams[0])
+
+    def replay():
+        q.launch(streams[1])
+
+    for rep in range(4):
+        for d in dsts:
+            d.zero_()
+        torch.cuda.synchronize()
+        for call in ((replay, eager) if graph_first else (eager, replay)):
+            call()
+        torch.cuda.synchronize()
+        for src, dst in zip(srcs, dsts):
+            part = [jobs[k] for k in (0, 23, 24, 35, 36, 40)]
+            data = []
+            for lg, _, so, _ in part:
+                x = src[so:so + (2 << lg)].cpu().numpy().astype(np.float64)
+                data.append(x[:1 << lg] + 1j * x[1 << lg:])
+            for (lg, inv, _, do), z in zip(part, data):
+                y = dst[do:do + (2 << lg)].cpu().numpy().astype(np.float64)
+                want = np.fft.ifft(z) if inv else np.fft.fft(z)
+                assert orc.rel_l2(y[:1 << lg] + 1j * y[1 << lg:], want) < fft_tol(1 << lg), (rep, lg, inv)
