@@ -83,9 +83,9 @@ int     pcx_plan_precision(pcx_plan_t plan);
  * pcx_plan_set_grid: workgroup caps of the column and row passes (0 = one per tile; the kernels
  *   loop over the rest; a plan starts with 2048 for tiles that fill a CU and none for smaller).
  *   pcx_plan_set_chunk: bytes of the intermediate of one chunk of a batch (0 = the default 2 GiB).
- *   pcx_plan_set_one_pass: calls of 48 or more 2^15-point FP32 transforms run in one pass (default
- *   on) or as the four-step (2^16 in natural order: calls of 180 or more run in one pass unless
- *   pcx_plan_set_shape named a split).
+ *   pcx_plan_set_one_pass: 2^15-point FP32 transforms run in one pass (default on; calls of less than
+ *   160 in place, inverse from a permuted order or of a queue do not) or as the four-step (2^16 in
+ *   natural order: calls of 180 or more run in one pass unless pcx_plan_set_shape named a split).
  *   pcx_plan_set_three_pass: natural-order transforms of 2^21 .. 2^24 points (FP64: 2^21 .. 2^23) run
  *   in three passes over the intermediate (default on) or as the four-step (the permuted orders
  *   always take the four-step). */

@@ -565,13 +565,16 @@ struct ExtTmp {
     int64_t bytes;
 };
 
-// Transforms from which a call of 2^15 points (FP64: 2^14) runs one workgroup per transform, and
-// from which 2^15 runs as k_dif before that; fewer transforms spread over the chip as small
-// four-step tiles.  2^15, forward, pack 8, four-step / k_dif / one pass, us: 1 transform 14.6 / 20.2 / 22.4,
-// 32 16.4 / 21.6 / -, 64 22.7 / 23.7 / 25.5, 256 51 / 41.9 / 36.9, 1024 248 / 188 / 159, 4096 (2^27
-// points) - / 710 / 546; bit_reversed 64 23.1 / 18.8 / 29.8, 256 51 / 43.9 / 40.6, 1024
-// 264 / 199 / 181.  FP64 2^14, four-step / one pass: 64 19.1 / 23.3, 256 48 / 32.3, 4096 790 / 484.
-constexpr int64_t kOnePassBatch = 160, kDifBatch = 48, kOnePassBatch64 = 96;
+// Transforms from which a call of 2^15 points (FP64: 2^14) runs one workgroup per transform; fewer
+// run as k_dif where that serves (out of place, forward or natural order) and spread over the chip
+// as small four-step tiles where it does not.  2^15, forward, pack 8, four-step / k_dif / one pass,
+// us: 1 transform 14.6 / 20.2 / 22.4, 32 16.4 / 21.6 / -, 64 22.7 / 23.7 / 25.5, 256 51 / 41.9 / 36.9,
+// 1024 248 / 188 / 159, 4096 (2^27 points) - / 710 / 546; bit_reversed 64 23.1 / 18.8 / 29.8, 256
+// 51 / 43.9 / 40.6, 1024 264 / 199 / 181.  FP64 2^14, four-step / one pass: 64 19.1 / 23.3, 256 48 / 32.3,
+// 4096 790 / 484.  (k_dif keeps the calls of less than 48 transforms although the four-step is faster
+// there: it needs no intermediate, so a fresh plan's first call may be captured, replays and calls on
+// several streams are independent, and the result does not depend on any of that.)
+constexpr int64_t kOnePassBatch = 160, kOnePassBatch64 = 96;
 
 // How many of a call's natural-order 2^15 / 2^16 transforms k_tile takes (one per CU and round, `ncu`
 // CUs): 2^16 in full rounds and a last one filled to more than 0.7, the others the four-step.
@@ -689,7 +692,7 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
 
     // ---- one pass, radix-R decimation in frequency + M-point Stockham (no intermediate)
     if constexpr (!F64)
-    if (p->use_one && p->precision == PCX_PREC_FP32 && batch >= kDifBatch && (const float*)dst != src && !src_offs &&
+    if (p->use_one && p->precision == PCX_PREC_FP32 && (const float*)dst != src && !src_offs &&
         (!inverse || p->order == PCX_ORDER_NORMAL)) {
         RowArgs a{};
         a.src = src, a.dst = dst, a.src_dist = src_dist, a.dst_dist = dst_dist;

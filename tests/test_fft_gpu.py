@@ -271,3 +271,41 @@ def test_shared_plan_on_two_streams(orc, pa):
         for b in (0, batch - 1):
             got = orc.from_packed(out[b * 2 * n:], n, n)
             assert orc.rel_l2(got, orc.fft64(xs[k][b].astype(np.complex128))) < fft_tol(n), (k, b)
+
+
+@pytest.mark.parametrize("order", ORDERS)
+@pytest.mark.parametrize("batch", [1, 9, 47])
+def test_one_pass_dif_first_call_in_a_capture(orc, pa, order, batch):
+    """Out of place, 2^15 points need no intermediate: the first calls of a fresh plan may be captured,
+    and replays run beside the plan's calls on another stream."""
+    import torch
+
+    n = 1 << 15
+    xs = [[orc.gen_normal(0x5EED0090 + 100 * k + b, n) for b in range(batch)] for k in range(2)]
+    srcs = [to_device(batch_buffer(x, n, 2 * n)) for x in xs]
+    dsts = [torch.zeros_like(s) for s in srcs]
+    back = torch.zeros_like(srcs[0])
+    unit = pa.fft_unit(n, order=order)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        unit.batch(dsts[0].data_ptr(), srcs[0].data_ptr(), batch, n, 2 * n, n, 2 * n)
+        if order == "normal":
+            unit.batch(back.data_ptr(), dsts[0].data_ptr(), batch, n, 2 * n, n, 2 * n, inverse=True)
+    side = torch.cuda.Stream()
+    slots = orc.slot_freq(order, n)
+    for rep in range(3):
+        for d in (*dsts, back):
+            d.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        unit.batch(dsts[1].data_ptr(), srcs[1].data_ptr(), batch, n, 2 * n, n, 2 * n, stream=side)
+        torch.cuda.synchronize()
+        for x, d in zip(xs, dsts):
+            out = d.cpu().numpy()
+            for b in sorted({0, batch - 1}):
+                got = orc.from_packed(out[b * 2 * n:], n, n)
+                assert orc.rel_l2(got, orc.fft64(x[b].astype(np.complex128))[slots]) < fft_tol(n), (rep, b)
+        if order == "normal":
+            got = orc.from_packed(back.cpu().numpy()[(batch - 1) * 2 * n:], n, n)
+            assert orc.rel_l2(got, xs[0][-1]) < 2 * fft_tol(n), rep
