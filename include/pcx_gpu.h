@@ -76,7 +76,8 @@ int     pcx_plan_precision(pcx_plan_t plan);
  * pcx_plan_set_shape: one of the instantiated N1 x N2 splits and tiles: column length
  *   2^n2_log2, `cols` columns per column tile, `rows` rows per row workgroup (0 = any; the first
  *   listed match wins, the default first; all 0: the default, and smaller tiles of its split for
- *   calls of few points, which a plan starts with).  Rebuilds the split's twiddle tables after a
+ *   calls of few points, which a plan starts with).  A named shape also turns off the one-pass forms
+ *   with one workgroup per transform (2^15, 2^16, FP64 2^14).  Rebuilds the split's twiddle tables after a
  *   device-wide synchronisation (every enqueued use of the old tables ends first).  Split-
  *   precision plans keep the default shape.
  * pcx_plan_shape: the current split and tiles (0s for a single-pass plan).

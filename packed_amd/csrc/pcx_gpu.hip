@@ -667,7 +667,9 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
     }
 
     // ---- one pass: one workgroup (or several, for small sizes) per group of whole transforms
-    const bool whole = p->use_one && p->precision == PCX_PREC_FP32 && batch >= (F64 ? kOnePassBatch64 : kOnePassBatch);
+    // (a named shape is the one that runs)
+    const bool whole = p->use_one && p->auto_shape && p->precision == PCX_PREC_FP32 &&
+                       batch >= (F64 ? kOnePassBatch64 : kOnePassBatch);
     if (!p->two_pass || whole) {
         RowArgsT<T> a{};
         a.src = src, a.dst = dst, a.src_dist = src_dist, a.dst_dist = dst_dist;

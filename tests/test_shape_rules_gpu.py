@@ -78,3 +78,40 @@ def test_whole_transforms_per_cu(orc, lg, rounds, rest, src_pack, dst_pack):
             assert orc.rel_l2(vec(dst, b, dst_pack), want) < tol, (inverse, b)
         gaps = dst.view(batch, dist)[:, 2 * n:]
         assert bool((gaps == (keep.view(batch, dist)[:, 2 * n:] if inplace else 7.0)).all())
+
+
+def _storages(n, batch, dtype, seed):
+    import torch
+
+    import packed_amd as pa
+
+    src, dst = pa.md_storage(n, batch, dtype=dtype), pa.md_storage(n, batch, dtype=dtype)
+    src.data.copy_(torch.randn(src.data.numel(), generator=torch.Generator("cuda").manual_seed(seed), device="cuda",
+                               dtype=src.data.dtype))
+    return src, dst
+
+
+@pytest.mark.parametrize("dtype,lg,batch,order", [("float64", 14, 97, "normal"), ("float64", 14, 97, "bit_reversed"),
+                                                  ("float32", 15, 161, "normal"), ("float32", 15, 161, "unordered")])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_named_shape_is_the_one_that_runs(dtype, lg, batch, order, inverse):
+    """A call that would run in one pass takes the four-step of a shape that was named (in place: the
+    out-of-place form of 2^15 follows the one-pass switch): within the bounds of both, not bit for bit,
+    and back to the first result with the automatic choice."""
+    import torch
+
+    import packed_amd as pa
+
+    n = 1 << lg
+    src, work = _storages(n, batch, dtype, lg + batch)
+    unit = pa.fft_unit(n, order=order, dtype=dtype)
+    outs = []
+    for shape in (0, 7, 0):
+        unit.set_shape(shape)
+        work.data.copy_(src.data)
+        unit.ifft(work) if inverse else unit(work)
+        outs.append(work.data.clone())
+    eps = 2.0 ** -23 if dtype == "float32" else 2.0 ** -52
+    diff = float(torch.linalg.norm((outs[0] - outs[1]).double()) / torch.linalg.norm(outs[0].double()))
+    assert 0 < diff < 4 * lg * eps
+    assert torch.equal(outs[0], outs[2])
