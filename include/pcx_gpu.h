@@ -82,7 +82,8 @@ int     pcx_plan_precision(pcx_plan_t plan);
  *   precision plans keep the default shape.
  * pcx_plan_shape: the current split and tiles (0s for a single-pass plan).
  * pcx_plan_set_grid: workgroup caps of the column and row passes (0 = one per tile; the kernels
- *   loop over the rest; a plan starts with 2048 for tiles that fill a CU and none for smaller).
+ *   loop over the rest; a plan starts with 2048 for tiles that fill a CU and none for smaller).  The
+ *   row cap also bounds the one-pass forms with one workgroup per transform (2^15, 2^16, FP64 2^14).
  *   pcx_plan_set_chunk: bytes of the intermediate of one chunk of a batch (0 = the default 2 GiB).
  *   pcx_plan_set_one_pass: 2^15-point FP32 transforms run in one pass (default on; calls of less than
  *   160 in place, inverse from a permuted order or of a queue do not) or as the four-step (2^16 in

@@ -642,6 +642,9 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
     else
         tw_row = p->tw_row, tw_col = p->tw_col, twl = p->twl, twh = p->twh;
 
+    // a cap of the row pass also holds for the workgroups that run whole transforms
+    const int64_t row_cap = std::max<int64_t>(p->grid_row, 0);
+
     // ---- one pass over a CU's registers and LDS
     if constexpr (!F64) {
         // offsets of multiples of 128 add under packs up to 128 and from N on
@@ -656,7 +659,7 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
                 t.a.src_offs = src_offs, t.a.dst_offs = dst_offs;
                 t.tw = p->tw_tile, t.tw128 = p->tw_tile + kTilePoints, t.twr = t.tw128 + kTileEdge;
                 t.src_sh = src_lp < p->lg, t.dst_sh = dst_lp < p->lg;
-                launch_tile(p->lg, t, p->ncu, st);
+                launch_tile(p->lg, t, row_cap > 0 ? std::min<int64_t>(row_cap, p->ncu) : p->ncu, st);
                 HIPCHK(hipGetLastError());
                 if (nb == batch)
                     return PCX_SUCCESS;
@@ -679,9 +682,9 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
         a.src_offs = src_offs, a.dst_offs = dst_offs;
         const int v = single_variant(inverse, p->order);
         if constexpr (F64)
-            (whole ? one_pass64_tab() : single64_tab()[p->lg - 1])[v](a, batch, 0, st);
+            (whole ? one_pass64_tab() : single64_tab()[p->lg - 1])[v](a, batch, whole ? row_cap : 0, st);
         else if (whole)
-            one_pass_tab()[v](a, batch, 0, st);
+            one_pass_tab()[v](a, batch, row_cap, st);
         else if (p->precision != PCX_PREC_FP32 && p->order == PCX_ORDER_NORMAL)
             single_mfma_tab()[p->precision - 1][p->lg - 4](a, batch, 0, st);
         else if (p->precision != PCX_PREC_FP32)

@@ -115,3 +115,31 @@ def test_named_shape_is_the_one_that_runs(dtype, lg, batch, order, inverse):
     diff = float(torch.linalg.norm((outs[0] - outs[1]).double()) / torch.linalg.norm(outs[0].double()))
     assert 0 < diff < 4 * lg * eps
     assert torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("dtype,lg,batch,order", [("float64", 14, 701, "normal"), ("float32", 15, 800, "bit_reversed"),
+                                                  ("float32", 16, 512, "normal")])
+def test_row_cap_holds_for_whole_transforms(dtype, lg, batch, order):
+    """The one-pass forms run under the caller's cap of row workgroups: 8 of them on 256 CUs take many
+    times as long, with the same result bit for bit."""
+    import torch
+
+    import packed_amd as pa
+
+    src, dst = _storages(1 << lg, batch, dtype, lg + batch)
+    unit = pa.fft_unit(1 << lg, order=order, dtype=dtype)
+    times, outs = [], []
+    for cap in (0, 8):
+        unit.set_grid(cap, cap)
+        best = float("inf")
+        for _ in range(3):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            unit(dst, src)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        times.append(best)
+        outs.append(dst.data.clone())
+    assert torch.equal(outs[0], outs[1])
+    assert times[1] > 4 * times[0], times
