@@ -85,9 +85,12 @@ int     pcx_plan_precision(pcx_plan_t plan);
  *   loop over the rest; a plan starts with 2048 for tiles that fill a CU and none for smaller).  The
  *   row cap also bounds the one-pass forms with one workgroup per transform (2^15, 2^16, FP64 2^14).
  *   pcx_plan_set_chunk: bytes of the intermediate of one chunk of a batch (0 = the default 2 GiB).
- *   pcx_plan_set_one_pass: 2^15-point FP32 transforms run in one pass (default on; calls of less than
- *   160 in place, inverse from a permuted order or of a queue do not) or as the four-step (2^16 in
- *   natural order: calls of 180 or more run in one pass unless pcx_plan_set_shape named a split).
+ *   pcx_plan_set_one_pass: one pass over memory where the plan has such a form (default on), or the
+ *   four-step: 2^15 FP32 (calls of less than 160 transforms in place, inverse from a permuted order or
+ *   of a queue take the four-step in any case); 2^16 FP32, natural order, whole sources, packs up to
+ *   128 or from 2^16 on (as many transforms as fill whole rounds of one per CU, and a last round
+ *   filled above 0.7; the others take the four-step and its intermediate); 2^14 FP64 (calls of 96 or
+ *   more).  Other plans refuse to turn it on.
  *   pcx_plan_set_three_pass: natural-order transforms of 2^21 .. 2^24 points (FP64: 2^21 .. 2^23) run
  *   in three passes over the intermediate (default on) or as the four-step (the permuted orders
  *   always take the four-step). */

@@ -204,9 +204,9 @@ struct pcx_plan_s {
     bool    auto_shape   = true; // no shape was chosen by the caller: calls of few points take small tiles
     int     nt_flags     = 0; // bit 0/1: streaming load/store of src/dst, bit 2/3: of the intermediate
     float2* tw_dif       = nullptr; // W_M for the one-pass k_dif kernel
-    // one-pass forms of 2^15 (FP64: 2^14) points (pcx_plan_set_one_pass): one workgroup per
-    // transform (W_N in tw_one), or k_dif
-    bool    use_one      = false;
+    // one-pass forms (pcx_plan_set_one_pass): one workgroup per transform of 2^15 (FP64: 2^14) points
+    // (W_N in tw_one), k_dif, k_tile
+    bool    use_one      = true;
     void*   tw_one       = nullptr;
     // natural-order 2^15 / 2^16: one pass over tiles held by one workgroup (k_tile): W_N in thread
     // order, W_128, W_(N/128)^(c t); one workgroup per CU
@@ -328,7 +328,6 @@ extern "C" int pcx_plan_create(int64_t fft_size, int64_t sub_size, int order, pc
         // transforms per four-step chunk: the intermediate holds one chunk
         p->chunk = std::max<int64_t>(1, kChunkBytes / (fft_size * 8));
         if (lg == kOnePassLog2) {
-            p->use_one      = true;
             const int64_t m = (int64_t)1 << dif_core_log2(order);
             if (he == hipSuccess)
                 he = hipMalloc(&p->tw_dif, sizeof(float2) * m);
@@ -448,7 +447,6 @@ extern "C" int pcx_plan_create_f64(int64_t fft_size, int64_t sub_size, int order
             he = gen_twiddles(p->twh64, fft_size, nl, nh, st);
         p->chunk = std::max<int64_t>(1, kChunkBytes / (fft_size * 16));
         if (lg == kOnePassLog2_64) {
-            p->use_one = true;
             if (he == hipSuccess)
                 he = hipMalloc(&p->tw_one, sizeof(double2) * fft_size);
             if (he == hipSuccess)
@@ -649,7 +647,7 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
     if constexpr (!F64) {
         // offsets of multiples of 128 add under packs up to 128 and from N on
         auto fits = [&](int lp) { return lp <= ilog2c(kTileEdge) || (lp >= p->lg && lp <= 27); };
-        if (p->tw_tile && p->auto_shape && (p->lg != kOnePassLog2 || p->use_one) && p->precision == PCX_PREC_FP32 &&
+        if (p->tw_tile && p->use_one && p->auto_shape && p->precision == PCX_PREC_FP32 &&
             src_size == n && fits(src_lp) && fits(dst_lp)) {
             if (const int64_t nb = tile_batch(p->lg, batch, p->ncu); nb > 0) {
                 TileArgs t{};
@@ -671,7 +669,7 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
 
     // ---- one pass: one workgroup (or several, for small sizes) per group of whole transforms
     // (a named shape is the one that runs)
-    const bool whole = p->use_one && p->auto_shape && p->precision == PCX_PREC_FP32 &&
+    const bool whole = p->tw_one && p->use_one && p->auto_shape && p->precision == PCX_PREC_FP32 &&
                        batch >= (F64 ? kOnePassBatch64 : kOnePassBatch);
     if (!p->two_pass || whole) {
         RowArgsT<T> a{};
@@ -697,7 +695,7 @@ int run_batch(pcx_plan_t p, int inverse, int normalized, T* dst, int64_t dst_pac
 
     // ---- one pass, radix-R decimation in frequency + M-point Stockham (no intermediate)
     if constexpr (!F64)
-    if (p->use_one && p->precision == PCX_PREC_FP32 && (const float*)dst != src && !src_offs &&
+    if (p->tw_dif && p->use_one && p->precision == PCX_PREC_FP32 && (const float*)dst != src && !src_offs &&
         (!inverse || p->order == PCX_ORDER_NORMAL)) {
         RowArgs a{};
         a.src = src, a.dst = dst, a.src_dist = src_dist, a.dst_dist = dst_dist;
@@ -956,7 +954,7 @@ extern "C" int pcx_plan_set_three_pass(pcx_plan_t p, int enable) {
 extern "C" int pcx_plan_set_one_pass(pcx_plan_t p, int enable) {
     if (!p)
         return fail(PCX_ERR_INVALID_ARGUMENT, "plan is null");
-    if (!p->tw_one || p->f64)
+    if (!p->tw_one && !p->tw_tile)
         return enable ? fail(PCX_ERR_UNSUPPORTED, "no one-pass kernel for fft_size " + s(p->n)) : PCX_SUCCESS;
     p->use_one = enable != 0;
     return PCX_SUCCESS;

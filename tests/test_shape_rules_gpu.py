@@ -143,3 +143,41 @@ def test_row_cap_holds_for_whole_transforms(dtype, lg, batch, order):
         outs.append(dst.data.clone())
     assert torch.equal(outs[0], outs[1])
     assert times[1] > 4 * times[0], times
+
+
+@pytest.mark.parametrize("dtype,lg,batch,order", [("float32", 15, 4, "normal"), ("float32", 15, 161, "unordered"),
+                                                  ("float32", 15, 800, "normal"), ("float32", 16, 200, "normal"),
+                                                  ("float64", 14, 97, "normal"), ("float64", 14, 97, "bit_reversed")])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_one_pass_switch(dtype, lg, batch, order, inverse):
+    """Every one-pass form (k_dif, one workgroup per transform, one per CU) against the four-step that the
+    switch selects: within the bounds of both, not bit for bit, and on again as before."""
+    import torch
+
+    import packed_amd as pa
+
+    n = 1 << lg
+    src, dst = _storages(n, batch, dtype, lg + batch)
+    unit = pa.fft_unit(n, order=order, dtype=dtype)
+    outs = []
+    for on in (None, False, True):
+        if on is not None:
+            unit.set_one_pass(on)
+        unit.ifft(dst, src) if inverse else unit(dst, src)
+        outs.append(dst.data.clone())
+    eps = 2.0 ** -23 if dtype == "float32" else 2.0 ** -52
+    diff = float(torch.linalg.norm((outs[0] - outs[1]).double()) / torch.linalg.norm(outs[0].double()))
+    assert 0 < diff < 4 * lg * eps
+    assert torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("dtype,lg,order", [("float32", 16, "bit_reversed"), ("float32", 17, "normal"),
+                                            ("float32", 14, "normal"), ("float64", 15, "normal")])
+def test_one_pass_switch_refused(dtype, lg, order):
+    """Plans without a one-pass form refuse to turn it on."""
+    import packed_amd as pa
+
+    unit = pa.fft_unit(1 << lg, order=order, dtype=dtype)
+    unit.set_one_pass(False)
+    with pytest.raises(pa.PcxError):
+        unit.set_one_pass(True)
