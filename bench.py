@@ -62,20 +62,48 @@ def profile_figure(name: str, key: str):
     return None
 
 
-def measured_traffic(log2n: int, batch: int, dtype: str = "float32"):
+def tile_share(log2n: int, batch: int, cus: int) -> int:
+    """Transforms of a natural-order FP32 batch that run with one transform per CU (the rule of
+    tile_batch in pcx_gpu.hip)."""
+    if log2n == 15:
+        return batch if batch > 3 * cus else 0
+    if log2n != 16:
+        return 0
+    last = batch % cus
+    return batch if 10 * last > 7 * cus else batch - last
+
+
+def forward_kernels(log2n: int, batch: int, dtype: str, precision: str, cus: int) -> str:
+    """The kernels that one forward step of the batch runs (natural order, split layout)."""
+    f64, split = dtype == "float64", precision != "fp32"
+    if log2n <= (13 if f64 else 14):
+        return "single pass k_row (one step = one launch)"
+    tiles = 0 if f64 or split else tile_share(log2n, batch, cus)
+    if tiles == batch:
+        return "k_tile, one transform per CU (one step = one launch)"
+    if not split and log2n == (14 if f64 else 15):
+        if batch >= (96 if f64 else 160):
+            return "single pass k_row, one transform per workgroup (one step = one launch)"
+        if not f64:
+            return "k_dif (one step = one launch)"
+    if not split and log2n >= 21:
+        return "three passes: k_col, k_col, k_row (one step = one launch of each)"
+    four = "four-step column pass k_col + row pass k_row"
+    if tiles:
+        return f"k_tile for {tiles} transforms, then {four} for {batch - tiles} (one step = one launch of each)"
+    return f"{four} (one step = one launch of each)"
+
+
+def traffic_profile(log2n: int, batch: int, dtype: str, cus: int) -> str:
+    tile = dtype == "float32" and tile_share(log2n, batch, cus) == batch
+    form = "tile_" if tile else "fourstep_" + ("" if dtype == "float32" else "f64_")
+    return f"fft_{form}n{1 << log2n}_b{batch}_hbm_traffic.md"
+
+
+def measured_traffic(log2n: int, batch: int, dtype: str, cus: int):
     """HBM bytes per step from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary of this
     workload (counters scaled by a plain copy of the same bytes); None for other shapes."""
-    return profile_figure(traffic_profile(log2n, batch, dtype), "traffic_bytes_per_step")
-
-
-def one_pass(log2n: int, dtype: str) -> bool:
-    """Sizes whose full batches run with one transform per CU (k_tile)."""
-    return dtype == "float32" and log2n in (15, 16)
-
-
-def traffic_profile(log2n: int, batch: int, dtype: str) -> str:
-    form = "tile_" if one_pass(log2n, dtype) else "fourstep_" + ("" if dtype == "float32" else "f64_")
-    return f"fft_{form}n{1 << log2n}_b{batch}_hbm_traffic.md"
+    return profile_figure(traffic_profile(log2n, batch, dtype, cus), "traffic_bytes_per_step")
 
 
 def time_steps(fn, steps, warmup):
@@ -264,7 +292,8 @@ def main():
         want = np.fft.fft(xc)
         yo = y[b * 2 * n:(b + 1) * 2 * n].cpu().numpy()
         errs.append(O.rel_l2(yo[:n] + 1j * yo[n:], want))
-    traffic = measured_traffic(args.log2n, batch, args.dtype) if args.precision == "fp32" else None
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    traffic = measured_traffic(args.log2n, batch, args.dtype, cus) if args.precision == "fp32" else None
     out = {
         "metric": ("C2C FFT GFLOP/s (5N\u00b7log2N) & %HBM peak, N=2^16 batch; MFMA-split vs FP32" if not f64
                    else "C2C FFT GFLOP/s (5N*log2N), N=2^16 batch 4096, FP64 split re/im"),
@@ -291,12 +320,10 @@ def main():
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic,
-            "traffic_source": (f"profiles/{traffic_profile(args.log2n, batch, args.dtype)}: "
+            "traffic_source": (f"profiles/{traffic_profile(args.log2n, batch, args.dtype, cus)}: "
                                "rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE of this workload, scaled by a plain copy"
                                if traffic else None),
-            "kernel": ("k_tile, one transform per CU (one step = one launch)"
-                       if args.precision == "fp32" and one_pass(args.log2n, args.dtype)
-                       else "four-step column pass k_col + row pass k_row (one step = one launch of each)"),
+            "kernel": forward_kernels(args.log2n, batch, args.dtype, args.precision, cus),
         },
         "inverse": {"ms": round(ms_inv, 4), "gflops": round(flops / (ms_inv * 1e-3) / 1e9, 1)},
         "bit_reversed": {"ms": round(ms_br, 4), "gflops": round(flops / (ms_br * 1e-3) / 1e9, 1),
