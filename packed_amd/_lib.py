@@ -135,8 +135,11 @@ def _current_stream():
     if not torch.cuda.is_available():
         raise RuntimeError("packed_amd needs a ROCm GPU: torch.cuda.is_available() is False")
     torch.cuda.current_stream()  # initialises the runtime
-    get, dev = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
-    _raw_stream = lambda: get(dev())  # noqa: E731
+    get, dev = (getattr(torch._C, name, None) for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+    if get and dev:
+        _raw_stream = lambda: get(dev())  # noqa: E731
+    else:  # a torch without these
+        _raw_stream = lambda: torch.cuda.current_stream().cuda_stream  # noqa: E731
     return _raw_stream()
 
 

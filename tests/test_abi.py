@@ -84,3 +84,25 @@ def test_f64_plan_validation():
     assert L.pcx_ifft_f64(None, 1, None, 4, None, 4, None) == _lib.ERR_INVALID_ARGUMENT
     assert L.pcx_fft_batch_f64(None, 0, 1, None, 4, 8, None, 4, 8, 4, 2, None) == _lib.ERR_INVALID_ARGUMENT
     assert L.pcx_plan_element_size(None) == 0
+
+
+@pytest.mark.parametrize("missing", [None, "_cuda_getCurrentRawStream", "_cuda_getDevice"])
+def test_current_stream_by_either_way(monkeypatch, missing):
+    """The stream of a call: torch's current one (looked up raw, or by the public call where torch has no
+    raw lookup), the one of a torch stream, or the handle itself."""
+    import types
+
+    import torch
+
+    from packed_amd import _lib
+
+    monkeypatch.setattr(_lib, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: types.SimpleNamespace(cuda_stream=700))
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda dev: 693 + dev, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 7, raising=False)
+    if missing:
+        monkeypatch.delattr(torch._C, missing)
+    assert [_lib.stream_ptr(None) for _ in range(2)] == [700, 700]
+    assert _lib.stream_ptr(types.SimpleNamespace(cuda_stream=5)) == 5
+    assert _lib.stream_ptr(11) == 11
