@@ -28,11 +28,6 @@ template<class T>
 __device__ __forceinline__ cx<T> cmul(cx<T> a, cx<T> w) {
     return {fmat(a.x, w.x, -a.y * w.y), fmat(a.x, w.y, a.y * w.x)};
 }
-// a * conj(w)
-template<class T>
-__device__ __forceinline__ cx<T> cmulc(cx<T> a, cx<T> w) {
-    return {fmat(a.x, w.x, a.y * w.y), fmat(a.y, w.x, -a.x * w.y)};
-}
 template<class T>
 __device__ __forceinline__ cx<T> cconj(cx<T> a) { return {a.x, -a.y}; }
 

@@ -24,7 +24,6 @@ constexpr int kMaxSinglePass   = 14; // N <= 16384 runs in one LDS-resident pass
 constexpr int kMaxLog2         = 24; // four-step limit: N2 <= 2048 columns, N1 <= 16384
 constexpr int kMaxSinglePass64 = 13; // FP64: N <= 8192 in one pass
 constexpr int kMaxLog2_64      = 23; // FP64 four-step limit
-constexpr int kDifLog2         = 15; // one-pass decimation-in-frequency size
 // Sizes beyond the single pass whose transform still fits a CU's LDS as one array (128 KiB): calls
 // of enough transforms run them in one pass, one workgroup per transform (one_pass_tab).
 constexpr int kOnePassLog2     = 15;
@@ -70,19 +69,20 @@ template<int LA, int G, int LD, int ST, int TW, bool UNI = (Plan<LA>::TA >= 64),
 void launch_row(const RowArgsT<T>& a, int64_t nrows, int64_t grid_cap, hipStream_t st) {
     constexpr int NT  = G * Plan<LA, false, T, PX>::TA;
     const int64_t nwg = fit_grid(grid8(even_grid((nrows + G - 1) / G, grid_cap)), NT);
-    // Pack 1 on both sides of a single pass: two 4-byte accesses at a stride of 8 bytes per element are
-    // bound by the rate of vector memory instructions, one of 8 bytes is not.  2^25 points forward, us:
-    // FP32 2^10 125 -> 107, 2^12 110 -> 100, 2^14 128 -> 113; FP64 2^11 211 -> 190, 2^14 288 -> 251, but
-    // 2^12 199 -> 204.  Permuted loads lose too (bit_reversed inverse 2^12 124 -> 169).  As a branch
-    // inside the kernels it cost the other packs 1 - 2 %.
-    if constexpr (UNI && PREC == PREC_FP32 && LD == LD_CONTIG && ST != ST_STRIDED && (PX & kPack1) == 0 &&
-                  !(sizeof(T) == 8 && LA == 12))
-        if (a.src_lp == 0 && a.dst_lp == 0) {
-            hipLaunchKernelGGL((k_row<LA, G, LD, ST, TW, UNI, ORD, PREC, T, PX | kPack1>), dim3((unsigned)nwg), dim3(NT),
-                               0, st, a);
-            return;
-        }
     hipLaunchKernelGGL((k_row<LA, G, LD, ST, TW, UNI, ORD, PREC, T, PX>), dim3((unsigned)nwg), dim3(NT), 0, st, a);
+}
+// Single passes.  Pack 1 on both sides: two 4-byte accesses at a stride of 8 bytes per element are
+// bound by the rate of vector memory instructions, one of 8 bytes is not.  2^25 points forward, us:
+// FP32 2^10 125 -> 107, 2^12 110 -> 100, 2^14 128 -> 113; FP64 2^11 211 -> 190, 2^14 288 -> 251, but
+// 2^12 199 -> 204.  Permuted loads lose too (bit_reversed inverse 2^12 124 -> 169).  As a branch
+// inside the kernels it cost the other packs 1 - 2 %.  (The four-step's rows read an intermediate of
+// pack N and have no such form.)
+template<int LA, int G, int LD, int ST, bool UNI, int ORD, class T = float, int PX = 0>
+void launch_single(const RowArgsT<T>& a, int64_t nrows, int64_t grid_cap, hipStream_t st) {
+    if constexpr (UNI && LD == LD_CONTIG && !(sizeof(T) == 8 && LA == 12))
+        if (a.src_lp == 0 && a.dst_lp == 0)
+            return launch_row<LA, G, LD, ST, 0, UNI, ORD, PREC_FP32, T, PX | kPack1>(a, nrows, grid_cap, st);
+    launch_row<LA, G, LD, ST, 0, UNI, ORD, PREC_FP32, T, PX>(a, nrows, grid_cap, st);
 }
 template<int LA, int C, int TW, int PREC = PREC_FP32, class T = float, int PX = 0>
 void launch_col(const ColArgsT<T>& a, int64_t grid_cap, hipStream_t st) {

@@ -12,9 +12,9 @@ constexpr std::array<RowLaunchT<double>, 5> single_set64() {
     using D            = double;
     constexpr int  G   = Plan<LA, false, D, PX>::TA >= 256 ? 1 : 256 / Plan<LA, false, D, PX>::TA;
     constexpr bool UNI = Plan<LA, false, D, PX>::TA >= 64;
-    return {&launch_row<LA, G, LD_CONTIG, ST_CONTIG, 0, UNI, 0, PREC_FP32, D, PX>,
-            &launch_row<LA, G, LD_CONTIG, ST_PERM, 0, UNI, ORD_BITREV, PREC_FP32, D, PX>, nullptr,
-            &launch_row<LA, G, LD_PERM, ST_CONTIG, 0, UNI, ORD_BITREV, PREC_FP32, D, PX>, nullptr};
+    return {&launch_single<LA, G, LD_CONTIG, ST_CONTIG, UNI, 0, D, PX>,
+            &launch_single<LA, G, LD_CONTIG, ST_PERM, UNI, ORD_BITREV, D, PX>, nullptr,
+            &launch_single<LA, G, LD_PERM, ST_CONTIG, UNI, ORD_BITREV, D, PX>, nullptr};
 }
 template<int... L>
 constexpr auto single_table64(std::integer_sequence<int, L...>) {

@@ -22,11 +22,11 @@ template<int LA, int PX = single_px<LA>()>
 constexpr RowSet single_set() {
     constexpr int  G   = Plan<LA, false, float, PX>::TA >= 256 ? 1 : 256 / Plan<LA, false, float, PX>::TA;
     constexpr bool UNI = Plan<LA, false, float, PX>::TA >= 64;
-    return {&launch_row<LA, G, LD_CONTIG, ST_CONTIG, 0, UNI, 0, PREC_FP32, float, PX>,
-            &launch_row<LA, G, LD_CONTIG, ST_PERM, 0, UNI, ORD_BITREV, PREC_FP32, float, PX>,
-            &launch_row<LA, G, LD_CONTIG, ST_PERM, 0, UNI, ORD_UNORD, PREC_FP32, float, PX>,
-            &launch_row<LA, G, LD_PERM, ST_CONTIG, 0, UNI, ORD_BITREV, PREC_FP32, float, PX>,
-            &launch_row<LA, G, LD_PERM, ST_CONTIG, 0, UNI, ORD_UNORD, PREC_FP32, float, PX>};
+    return {&launch_single<LA, G, LD_CONTIG, ST_CONTIG, UNI, 0, float, PX>,
+            &launch_single<LA, G, LD_CONTIG, ST_PERM, UNI, ORD_BITREV, float, PX>,
+            &launch_single<LA, G, LD_CONTIG, ST_PERM, UNI, ORD_UNORD, float, PX>,
+            &launch_single<LA, G, LD_PERM, ST_CONTIG, UNI, ORD_BITREV, float, PX>,
+            &launch_single<LA, G, LD_PERM, ST_CONTIG, UNI, ORD_UNORD, float, PX>};
 }
 template<int... L>
 constexpr auto single_table(std::integer_sequence<int, L...>) {
