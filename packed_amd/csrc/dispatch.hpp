@@ -282,7 +282,6 @@ const std::array<AcrossLaunch64, kMaxAcross64>& across64_tab(); // index LA-1
 // ---- k_tile.hip: natural-order transforms of 2^15 / 2^16 points, `grid` workgroups
 constexpr int kCuTileMinLog2 = 15, kCuTileMaxLog2 = 16;
 void launch_tile(int lg, const TileArgs& a, int64_t grid, hipStream_t st);
-void launch_tile_twiddles(float2* t, int lg, hipStream_t st);
 
 // ---- launchers of the remaining kernels (k_misc.hip)
 void launch_queue(const QueueArgs& a, int grid, hipStream_t st);

@@ -4,7 +4,7 @@
 //          transform), pass B of the forward four-step and pass 1 of the inverse four-step.
 //  k_col   FFTs down columns of a row-major tile (stride N1): pass A of the forward four-step and
 //          pass 2 of the inverse.  A wavefront reads and writes C consecutive floats per row.
-//  k_twiddles, k_generate  plan-time twiddle tables (FP64, rounded to FP32) and seeded inputs.
+//  k_twiddles, k_generate  twiddle tables (FP64, rounded to FP32) and seeded inputs.
 //
 // Inverse transforms run as conj(FFT(conj(x))): conj_in / conj_out negate imaginary parts at
 // load and store, so every kernel only implements the forward butterflies.
@@ -1240,15 +1240,18 @@ __global__ __launch_bounds__((C * Plan<LA, false, T>::TA)) void k_across(AcrossA
     }
 }
 
+// W_M^k (evaluated in FP64, rounded to T)
+template<class T>
+__device__ __forceinline__ vec2<T> twiddle(int64_t k, int64_t M) {
+    double s, c;
+    sincospi(-2.0 * (double)k / (double)M, &s, &c);
+    return vec2<T>{(T)c, (T)s};
+}
 template<class T>
 __global__ void k_twiddles(vec2<T>* t, int64_t M, int64_t stride, int64_t count) {
     int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= count)
-        return;
-    int64_t k = (e * stride) % M;
-    double  s, c;
-    sincospi(-2.0 * (double)k / (double)M, &s, &c);
-    t[e] = vec2<T>{(T)c, (T)s};
+    if (e < count)
+        t[e] = twiddle<T>((e * stride) % M, M);
 }
 
 // Seeded inputs: output k of splitmix64(seed) is mix(seed + (k+1)*gamma), so element i uses

@@ -9,8 +9,5 @@ void launch_tile(int lg, const TileArgs& a, int64_t grid, hipStream_t st) {
     const auto f   = lg == 15 ? (one ? k_tile<2, true> : k_tile<2, false>) : (one ? k_tile<4, true> : k_tile<4, false>);
     hipLaunchKernelGGL(f, g, dim3(kTileThreads), 0, st, a);
 }
-void launch_tile_twiddles(float2* t, int lg, hipStream_t st) {
-    hipLaunchKernelGGL(k_tile_twiddles, dim3((tile_table((1 << lg) / kTilePoints) + 255) / 256), dim3(256), 0, st, t, lg);
-}
 
 } // namespace pcxd

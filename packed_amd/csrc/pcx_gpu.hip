@@ -98,6 +98,32 @@ hipError_t gen_twiddles(V* t, int64_t M, int64_t stride, int64_t count, hipStrea
     return hipGetLastError();
 }
 
+// Twiddle tables filled by one launch: table k holds W_m^(stride e) for e < end[k] - end[k - 1], or
+// (m = 0) the array that k_tile reads.
+constexpr int kMaxTables = 10;
+template<class T>
+struct TablesArgs {
+    vec2<T>* t[kMaxTables];
+    int64_t  m[kMaxTables], stride[kMaxTables], end[kMaxTables];
+    int      count, lg;
+};
+template<class T>
+__global__ __launch_bounds__(256) void k_tables(TablesArgs<T> a) {
+    int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int     k = 0;
+    while (k < a.count && e >= a.end[k])
+        ++k;
+    if (k == a.count)
+        return;
+    if (k > 0)
+        e -= a.end[k - 1];
+    if constexpr (sizeof(T) == 4)
+        if (a.m[k] == 0) {
+            a.t[k][e] = tile_twiddle((int)e, a.lg);
+            return;
+        }
+    a.t[k][e] = twiddle<T>((e * a.stride[k]) % a.m[k], a.m[k]);
+}
 
 // ---------------------------------------------------------------- shape lookup
 template<class T>
@@ -183,6 +209,7 @@ struct pcx_plan_s {
     int     order = 0;
     bool    two_pass = false;
     int     n1_lg = 0, n2_lg = 0; // N = N1 * N2, N1 contiguous (row) length, N2 column length
+    void*   tables = nullptr;     // the allocation that holds every table below
     float2* tw_row = nullptr;     // W_N (single pass) or W_N1
     float2* tw_col = nullptr;     // W_N2
     float2* twl    = nullptr;     // W_N^e, e < 2^tw_ls
@@ -236,53 +263,83 @@ namespace {
 // in one chunk; a 288 GB part holds it several times over).
 constexpr int64_t kChunkBytes = (int64_t)2048 << 20;
 
-// Twiddle tables of a four-step FP32 plan for its shape's N1 x N2 split (W_N1, W_N2) and the
-// pass tables W_N = lo[e mod 2^ls] * hi[e >> ls].
-// Tables of the three-pass form: stage tables W_N2, W_Nb, W_Na and the two-level W_N1 table of
-// pass 2 (the W_N pass table is the four-step one).  T = float or double.
+// The twiddle tables of a plan for its N1 x N2 split, in one allocation filled by one launch (a 2^15
+// plan has seven tables: 32 us to create with an allocation and a launch for each, 16 so).  A
+// plan that has tables keeps them if the new ones cannot be made; its callers see to it that no
+// enqueued work uses the old ones.
 template<class T>
-hipError_t three_pass_tables(pcx_plan_t p, hipStream_t st) {
-    using V                   = vec2<T>;
-    const ThreePassT<T>* tp   = three_of<T>(p->lg);
-    if (!tp)
-        return hipSuccess;
-    const int     l1 = p->lg - tp->n2_lg;
-    const int64_t n1 = (int64_t)1 << l1;
-    p->tw_ls1        = (l1 + 1) / 2;
-    const int64_t len[5]   = {(int64_t)1 << tp->n2_lg, (int64_t)1 << kThreeNbLog2, (int64_t)1 << tp->na_lg,
-                              (int64_t)1 << p->tw_ls1, n1 >> p->tw_ls1};
-    const int64_t m[5]     = {len[0], len[1], len[2], n1, n1};
-    const int64_t stride[5] = {1, 1, 1, 1, len[3]};
-    hipError_t    he       = hipSuccess;
-    for (int k = 0; k < 5 && he == hipSuccess; ++k) {
-        he = hipMalloc(&p->tw3[k], sizeof(V) * len[k]);
-        if (he == hipSuccess)
-            he = gen_twiddles((V*)p->tw3[k], m[k], stride[k], len[k], st);
+hipError_t plan_tables(pcx_plan_t p, hipStream_t st) {
+    using V            = vec2<T>;
+    constexpr bool F64 = sizeof(T) == 8;
+    TablesArgs<T>  a{};
+    void**         place[kMaxTables];
+    int64_t        offset[kMaxTables], bytes = 0;
+    auto           add = [&](auto** table, int64_t m, int64_t stride, int64_t count) {
+        const int k = a.count++;
+        place[k]    = (void**)table;
+        offset[k]   = bytes;
+        a.m[k] = m, a.stride[k] = stride, a.end[k] = (k > 0 ? a.end[k - 1] : 0) + count;
+        bytes += (count * (int64_t)sizeof(V) + 255) & ~(int64_t)255;
+    };
+    V **row, **col, **lo, **hi;
+    if constexpr (F64)
+        row = &p->tw64_row, col = &p->tw64_col, lo = &p->twl64, hi = &p->twh64;
+    else
+        row = &p->tw_row, col = &p->tw_col, lo = &p->twl, hi = &p->twh;
+    const int64_t n = p->n;
+    if (!p->two_pass) {
+        add(row, n, 1, n);
+    } else {
+        // W_N1, W_N2 and the pass tables W_N = lo[e mod 2^ls] * hi[e >> ls]
+        const int64_t n1 = (int64_t)1 << p->n1_lg, n2 = (int64_t)1 << p->n2_lg, nl = (int64_t)1 << p->tw_ls;
+        add(row, n1, 1, n1);
+        add(col, n2, 1, n2);
+        add(lo, n, 1, nl);
+        add(hi, n, nl, n / nl);
+        // the three-pass form: stage tables W_N2, W_Nb, W_Na and the two-level W_N1 table of pass 2
+        if (const ThreePassT<T>* tp = three_of<T>(p->lg)) {
+            const int l1 = p->lg - tp->n2_lg, ls = (l1 + 1) / 2;
+            add(&p->tw3[0], (int64_t)1 << tp->n2_lg, 1, (int64_t)1 << tp->n2_lg);
+            add(&p->tw3[1], (int64_t)1 << kThreeNbLog2, 1, (int64_t)1 << kThreeNbLog2);
+            add(&p->tw3[2], (int64_t)1 << tp->na_lg, 1, (int64_t)1 << tp->na_lg);
+            add(&p->tw3[3], (int64_t)1 << l1, 1, (int64_t)1 << ls);
+            add(&p->tw3[4], (int64_t)1 << l1, (int64_t)1 << ls, (int64_t)1 << (l1 - ls));
+            p->tw_ls1 = ls;
+        }
+        if (p->lg == (F64 ? kOnePassLog2_64 : kOnePassLog2))
+            add(&p->tw_one, n, 1, n);
+        if constexpr (!F64) {
+            const int64_t m = (int64_t)1 << dif_core_log2(p->order);
+            if (p->lg == kOnePassLog2)
+                add(&p->tw_dif, m, 1, m);
+            if (p->order == PCX_ORDER_NORMAL && p->lg >= kCuTileMinLog2 && p->lg <= kCuTileMaxLog2)
+                add(&p->tw_tile, 0, 0, tile_table((int)(n / kTilePoints)));
+        }
+    }
+    char*      block = nullptr;
+    hipError_t he    = hipMalloc(&block, bytes);
+    if (he != hipSuccess)
+        return he;
+    for (int k = 0; k < a.count; ++k)
+        a.t[k] = reinterpret_cast<V*>(block + offset[k]);
+    a.lg = p->lg;
+    if (a.count == 1) { // 14.3 us for a single pass, 15.3 with k_tables
+        he = gen_twiddles(a.t[0], a.m[0], a.stride[0], a.end[0], st);
+    } else {
+        hipLaunchKernelGGL(k_tables<T>, dim3((unsigned)((a.end[a.count - 1] + 255) / 256)), dim3(256), 0, st, a);
+        he = hipGetLastError();
     }
     if (he == hipSuccess)
-        p->use_three = true;
-    return he;
-}
-
-hipError_t fourstep_tables(pcx_plan_t p, hipStream_t st) {
-    const int64_t n1 = (int64_t)1 << p->n1_lg, n2 = (int64_t)1 << p->n2_lg;
-    const int64_t nl = (int64_t)1 << p->tw_ls, nh = p->n >> p->tw_ls;
-    hipError_t    he = hipMalloc(&p->tw_row, sizeof(float2) * n1);
-    if (he == hipSuccess)
-        he = hipMalloc(&p->tw_col, sizeof(float2) * n2);
-    if (he == hipSuccess && !p->twl)
-        he = hipMalloc(&p->twl, sizeof(float2) * nl);
-    if (he == hipSuccess && !p->twh)
-        he = hipMalloc(&p->twh, sizeof(float2) * nh);
-    if (he == hipSuccess)
-        he = gen_twiddles(p->tw_row, n1, 1, n1, st);
-    if (he == hipSuccess)
-        he = gen_twiddles(p->tw_col, n2, 1, n2, st);
-    if (he == hipSuccess)
-        he = gen_twiddles(p->twl, p->n, 1, nl, st);
-    if (he == hipSuccess)
-        he = gen_twiddles(p->twh, p->n, nl, nh, st);
-    return he;
+        he = hipStreamSynchronize(st);
+    if (he != hipSuccess) {
+        (void)hipFree(block);
+        return he;
+    }
+    for (int k = 0; k < a.count; ++k)
+        *place[k] = a.t[k];
+    (void)hipFree(p->tables);
+    p->tables = block;
+    return hipSuccess;
 }
 
 } // namespace
@@ -309,12 +366,7 @@ extern "C" int pcx_plan_create(int64_t fft_size, int64_t sub_size, int order, pc
     p->n     = fft_size;
     p->lg    = lg;
     p->order = order;
-    hipError_t he = hipSuccess;
-    if (lg <= kMaxSinglePass) {
-        he = hipMalloc(&p->tw_row, sizeof(float2) * fft_size);
-        if (he == hipSuccess)
-            he = gen_twiddles(p->tw_row, fft_size, 1, fft_size, st);
-    } else {
+    if (lg > kMaxSinglePass) {
         p->two_pass = true;
         p->shape    = default_shape(lg, order);
         if (!p->shape) {
@@ -324,41 +376,21 @@ extern "C" int pcx_plan_create(int64_t fft_size, int64_t sub_size, int order, pc
         p->n2_lg = p->shape->n2;
         p->n1_lg = p->shape->n1;
         p->tw_ls = (lg + 1) / 2;
-        he       = fourstep_tables(p, st);
         // transforms per four-step chunk: the intermediate holds one chunk
         p->chunk = std::max<int64_t>(1, kChunkBytes / (fft_size * 8));
-        if (lg == kOnePassLog2) {
-            const int64_t m = (int64_t)1 << dif_core_log2(order);
-            if (he == hipSuccess)
-                he = hipMalloc(&p->tw_dif, sizeof(float2) * m);
-            if (he == hipSuccess)
-                he = gen_twiddles(p->tw_dif, m, 1, m, st);
-            if (he == hipSuccess)
-                he = hipMalloc(&p->tw_one, sizeof(float2) * fft_size);
-            if (he == hipSuccess)
-                he = gen_twiddles((float2*)p->tw_one, fft_size, 1, fft_size, st);
-        }
-        if (he == hipSuccess && order == PCX_ORDER_NORMAL && lg >= kCuTileMinLog2 && lg <= kCuTileMaxLog2) {
-            int dev = 0;
-            he = hipGetDevice(&dev);
-            if (he == hipSuccess)
-                he = hipDeviceGetAttribute(&p->ncu, hipDeviceAttributeMultiprocessorCount, dev);
-            if (he == hipSuccess)
-                he = hipMalloc(&p->tw_tile, sizeof(float2) * tile_table((int)(fft_size / kTilePoints)));
-            if (he == hipSuccess) {
-                launch_tile_twiddles(p->tw_tile, lg, st);
-                he = hipGetLastError();
-            }
-        }
-        // three passes are the default: 2^21 / 2^22 / 2^23 / 2^24 in 2.74 / 2.83 / 2.93 /
-        // 2.95 ms per 2 GiB forward against 3.03 / 3.67 / 4.45 / 6.00 with the four-step
-        if (he == hipSuccess)
-            he = three_pass_tables<float>(p, st);
-        if (he == hipSuccess)
-            he = hipEventCreateWithFlags(&p->tmp_ev, hipEventDisableTiming);
     }
-    if (he == hipSuccess)
-        he = hipStreamSynchronize(st);
+    // three passes are the default where they exist: 2^21 / 2^22 / 2^23 / 2^24 in 2.74 / 2.83 / 2.93 /
+    // 2.95 ms per 2 GiB forward against 3.03 / 3.67 / 4.45 / 6.00 with the four-step
+    hipError_t he = plan_tables<float>(p, st);
+    p->use_three  = p->tw3[0] != nullptr;
+    if (he == hipSuccess && p->tw_tile) {
+        int dev = 0;
+        he      = hipGetDevice(&dev);
+        if (he == hipSuccess)
+            he = hipDeviceGetAttribute(&p->ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    }
+    if (he == hipSuccess && p->two_pass)
+        he = hipEventCreateWithFlags(&p->tmp_ev, hipEventDisableTiming);
     if (he != hipSuccess) {
         pcx_plan_destroy(p);
         return fail(PCX_ERR_HIP, std::string("plan setup: ") + hipGetErrorString(he));
@@ -373,20 +405,8 @@ extern "C" int pcx_plan_destroy(pcx_plan_t p) {
     // the intermediate may still be in use by enqueued work
     if (p->tmp_ev && p->tmp_used)
         (void)hipEventSynchronize(p->tmp_ev);
-    (void)hipFree(p->tw_row);
-    (void)hipFree(p->tw_col);
-    (void)hipFree(p->twl);
-    (void)hipFree(p->twh);
+    (void)hipFree(p->tables);
     (void)hipFree(p->tmp);
-    (void)hipFree(p->tw_dif);
-    (void)hipFree(p->tw_one);
-    (void)hipFree(p->tw_tile);
-    for (void* t : p->tw3)
-        (void)hipFree(t);
-    (void)hipFree(p->tw64_row);
-    (void)hipFree(p->tw64_col);
-    (void)hipFree(p->twl64);
-    (void)hipFree(p->twh64);
     if (p->tmp_ev)
         (void)hipEventDestroy(p->tmp_ev);
     delete p;
@@ -417,48 +437,18 @@ extern "C" int pcx_plan_create_f64(int64_t fft_size, int64_t sub_size, int order
     p->lg    = lg;
     p->order = order;
     p->f64   = true;
-    hipError_t he = hipSuccess;
-    if (lg <= kMaxSinglePass64) {
-        he = hipMalloc(&p->tw64_row, sizeof(double2) * fft_size);
-        if (he == hipSuccess)
-            he = gen_twiddles(p->tw64_row, fft_size, 1, fft_size, st);
-    } else {
+    if (lg > kMaxSinglePass64) {
         p->two_pass = true;
         p->shape64  = default_shape64(lg, order);
         p->n1_lg    = p->shape64->n1;
         p->n2_lg    = p->shape64->n2;
         p->tw_ls    = (lg + 1) / 2;
-        int64_t n1 = (int64_t)1 << p->n1_lg, n2 = (int64_t)1 << p->n2_lg;
-        int64_t nl = (int64_t)1 << p->tw_ls, nh = fft_size >> p->tw_ls;
-        he = hipMalloc(&p->tw64_row, sizeof(double2) * n1);
-        if (he == hipSuccess)
-            he = hipMalloc(&p->tw64_col, sizeof(double2) * n2);
-        if (he == hipSuccess)
-            he = hipMalloc(&p->twl64, sizeof(double2) * nl);
-        if (he == hipSuccess)
-            he = hipMalloc(&p->twh64, sizeof(double2) * nh);
-        if (he == hipSuccess)
-            he = gen_twiddles(p->tw64_row, n1, 1, n1, st);
-        if (he == hipSuccess)
-            he = gen_twiddles(p->tw64_col, n2, 1, n2, st);
-        if (he == hipSuccess)
-            he = gen_twiddles(p->twl64, fft_size, 1, nl, st);
-        if (he == hipSuccess)
-            he = gen_twiddles(p->twh64, fft_size, nl, nh, st);
-        p->chunk = std::max<int64_t>(1, kChunkBytes / (fft_size * 16));
-        if (lg == kOnePassLog2_64) {
-            if (he == hipSuccess)
-                he = hipMalloc(&p->tw_one, sizeof(double2) * fft_size);
-            if (he == hipSuccess)
-                he = gen_twiddles((double2*)p->tw_one, fft_size, 1, fft_size, st);
-        }
-        if (he == hipSuccess)
-            he = three_pass_tables<double>(p, st);
-        if (he == hipSuccess)
-            he = hipEventCreateWithFlags(&p->tmp_ev, hipEventDisableTiming);
+        p->chunk    = std::max<int64_t>(1, kChunkBytes / (fft_size * 16));
     }
-    if (he == hipSuccess)
-        he = hipStreamSynchronize(st);
+    hipError_t he = plan_tables<double>(p, st);
+    p->use_three  = p->tw3[0] != nullptr;
+    if (he == hipSuccess && p->two_pass)
+        he = hipEventCreateWithFlags(&p->tmp_ev, hipEventDisableTiming);
     if (he != hipSuccess) {
         pcx_plan_destroy(p);
         return fail(PCX_ERR_HIP, std::string("plan setup: ") + hipGetErrorString(he));
@@ -510,45 +500,38 @@ extern "C" int     pcx_plan_order(pcx_plan_t p) { return p ? p->order : -1; }
 
 namespace {
 
-// Switches a four-step plan to another instantiated shape, rebuilding the W_N1 / W_N2 tables
-// when the split changes (the pass tables W_N do not depend on the split).
+// Moves a four-step plan to the split of another instantiated shape: the tables follow the split.
+template<class T>
+int plan_apply_split(pcx_plan_t p, int n1_lg, int n2_lg) {
+    if (n1_lg == p->n1_lg && n2_lg == p->n2_lg)
+        return PCX_SUCCESS;
+    // every enqueued use of the old tables must end
+    HIPCHK(hipDeviceSynchronize());
+    hipStream_t st = nullptr;
+    HIPCHK(setup_stream(&st));
+    std::swap(p->n1_lg, n1_lg), std::swap(p->n2_lg, n2_lg);
+    const hipError_t he = plan_tables<T>(p, st);
+    if (he != hipSuccess)
+        p->n1_lg = n1_lg, p->n2_lg = n2_lg; // the tables are still the old split's
+    HIPCHK(he);
+    return PCX_SUCCESS;
+}
+
 int plan_apply_shape(pcx_plan_t p, const FourStep* sh) {
     if (!p->two_pass || p->f64 || !sh || sh->lg != p->lg)
         return fail(PCX_ERR_INVALID_ARGUMENT, "shape does not match the plan");
-    if (sh->n1 != p->n1_lg || sh->n2 != p->n2_lg) {
-        // the W_N1 / W_N2 tables follow the split; every enqueued use of the old ones must end
-        HIPCHK(hipDeviceSynchronize());
-        HIPCHK(hipFree(p->tw_row));
-        HIPCHK(hipFree(p->tw_col));
-        p->tw_row = p->tw_col = nullptr;
-        p->n1_lg = sh->n1, p->n2_lg = sh->n2;
-        hipStream_t st = nullptr;
-        HIPCHK(setup_stream(&st));
-        HIPCHK(fourstep_tables(p, st));
-        HIPCHK(hipStreamSynchronize(st));
-    }
-    p->shape = sh, p->n1_lg = sh->n1, p->n2_lg = sh->n2;
+    if (int e = plan_apply_split<float>(p, sh->n1, sh->n2))
+        return e;
+    p->shape = sh;
     return PCX_SUCCESS;
 }
 
 int plan_apply_shape64(pcx_plan_t p, const FourStepT<double>* sh) {
     if (!p->two_pass || !p->f64 || !sh || sh->lg != p->lg)
         return fail(PCX_ERR_INVALID_ARGUMENT, "shape does not match the plan");
-    if (sh->n1 != p->n1_lg || sh->n2 != p->n2_lg) {
-        HIPCHK(hipDeviceSynchronize());
-        HIPCHK(hipFree(p->tw64_row));
-        HIPCHK(hipFree(p->tw64_col));
-        p->tw64_row = p->tw64_col = nullptr;
-        const int64_t n1 = (int64_t)1 << sh->n1, n2 = (int64_t)1 << sh->n2;
-        hipStream_t   st = nullptr;
-        HIPCHK(setup_stream(&st));
-        HIPCHK(hipMalloc(&p->tw64_row, sizeof(double2) * n1));
-        HIPCHK(hipMalloc(&p->tw64_col, sizeof(double2) * n2));
-        HIPCHK(gen_twiddles(p->tw64_row, n1, 1, n1, st));
-        HIPCHK(gen_twiddles(p->tw64_col, n2, 1, n2, st));
-        HIPCHK(hipStreamSynchronize(st));
-    }
-    p->shape64 = sh, p->n1_lg = sh->n1, p->n2_lg = sh->n2;
+    if (int e = plan_apply_split<double>(p, sh->n1, sh->n2))
+        return e;
+    p->shape64 = sh;
     return PCX_SUCCESS;
 }
 

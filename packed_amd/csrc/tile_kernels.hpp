@@ -35,33 +35,24 @@ constexpr int kTileThreads = 1024, kTileEdge = 128, kTilePoints = kTileEdge * kT
 
 struct TileArgs {
     RowArgs       a;     // one row per transform; src_size = N
-    const float2* tw;    // W_N^(c k2) at [slot][thread] (k_tile_twiddles)
+    const float2* tw;    // W_N^(c k2) at [slot][thread] (tile_twiddle)
     const float2* tw128; // W_128
     const float2* twr;   // W_(128R)^(c t) at [t][c] (and W_(128R)^(T k2) at [T][k2])
     int           src_sh, dst_sh; // 1 for packs up to 128, 0 for packs >= N: poff(128 x) = 128 x << sh
 };
 
-// Tables of a plan of 2^lg points in one array: W_N^(c k2) at [slot][thread], slot = 8m + r,
-// thread = 128 j8 + c, k2 = j8 + 8m + 16r; then W_128; then W_(128R)^(c t) at [t][c].
+// k_tile's tables in one array: W_N^(c k2) at [slot][thread], slot = 8m + r, thread = 128 j8 + c,
+// k2 = j8 + 8m + 16r; then W_128; then W_(128R)^(c t) at [t][c].  Entry e of 2^lg points' array:
 constexpr int tile_table(int r) { return kTilePoints + kTileEdge * (1 + r); }
-static __global__ __launch_bounds__(256) void k_tile_twiddles(float2* t, int lg) {
-    const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+__device__ __forceinline__ float2 tile_twiddle(int e, int lg) {
     const int r = (1 << lg) / kTilePoints, f = e - kTilePoints;
-    if (e >= tile_table(r))
-        return;
-    int x, n; // W_n^x
     if (f < 0) {
         const int th = e & 1023, slot = e >> 10;
-        x            = (th & 127) * ((th >> 7) + 8 * (slot >> 3) + 16 * (slot & 7));
-        n            = 1 << lg;
-    } else if (f < kTileEdge) {
-        x = f, n = kTileEdge;
-    } else {
-        x = (f % kTileEdge) * (f / kTileEdge - 1), n = kTileEdge * r;
+        return twiddle<float>((th & 127) * ((th >> 7) + 8 * (slot >> 3) + 16 * (slot & 7)), 1 << lg);
     }
-    double s, c;
-    sincospi(-2.0 * (double)x / (double)n, &s, &c);
-    t[e] = float2{(float)c, (float)s};
+    if (f < kTileEdge)
+        return twiddle<float>(f, kTileEdge);
+    return twiddle<float>((f % kTileEdge) * (f / kTileEdge - 1), kTileEdge * r);
 }
 
 // LDS floats.  Exchanges of a tile: re and im arrays of 128 rows; columns unpadded, rows at a stride

@@ -181,3 +181,25 @@ def test_one_pass_switch_refused(dtype, lg, order):
     unit.set_one_pass(False)
     with pytest.raises(pa.PcxError):
         unit.set_one_pass(True)
+
+
+@pytest.mark.parametrize("dtype,lg,other", [("float32", 15, 17), ("float32", 16, 17), ("float64", 14, 15)])
+def test_one_pass_tables_cost_no_plan_time(dtype, lg, other):
+    """Plans with tables of one-pass forms are made as fast as the next size's without (the quickest of
+    many plans made in turn; the tables of a plan are filled by one launch)."""
+    import time
+
+    import torch
+
+    import packed_amd as pa
+
+    torch.zeros(1, device="cuda")
+    times = {lg: [], other: []}
+    for _ in range(200):
+        for k in times:
+            start = time.perf_counter()
+            unit = pa.fft_unit(1 << k, dtype=dtype)
+            times[k].append(time.perf_counter() - start)
+            del unit
+    a, b = min(times[lg]), min(times[other])
+    assert a < 1.12 * b, (a, b)
