@@ -237,3 +237,24 @@ def test_replay_and_eager_pass_on_two_streams(orc, pa, graph_first):
                 y = dst[do:do + (2 << lg)].cpu().numpy().astype(np.float64)
                 want = np.fft.ifft(z) if inv else np.fft.fft(z)
                 assert orc.rel_l2(y[:1 << lg] + 1j * y[1 << lg:], want) < fft_tol(1 << lg), (rep, lg, inv)
+
+
+def test_tuning_file_of_the_earlier_queue(orc, pa, tmp_path):
+    """A file written when the persistent launch took sizes to 2^20: its classes above 2^14 are full-chip
+    launches in any case, its workgroup count is cut to the launch's own, its shapes are taken."""
+    import torch
+
+    jobs, total, buf, data = _case(orc, 10)
+    src = torch.from_numpy(buf).cuda()
+    dst = torch.zeros_like(src)
+    cache = tmp_path / "tune.txt"
+    cache.write_text("grouped 9 0\ngrouped 15 0\ngrouped 15 1\ngrouped 18 1\ngrouped 20 0\ngrouped 20 1\nqueue_grid 4096\n"
+                     "group 20 0 10 16 16 2048 2048\ngroup 20 1 10 16 16 1024 1024\ngroup 18 1 9 32 32 0 0\n"
+                     "group 15 0 7 32 64 1024 1024\ngroup 15 1 7 64 128 0 0\n")
+    text = cache.read_text()
+    q = pa.fft_queue(jobs)
+    q.autotune(dst.data_ptr(), src.data_ptr(), str(cache))
+    q.exec(dst.data_ptr(), src.data_ptr())
+    torch.cuda.synchronize()
+    _check(orc, jobs, data, dst.cpu().numpy())
+    assert cache.read_text() == text

@@ -203,3 +203,25 @@ def test_one_pass_tables_cost_no_plan_time(dtype, lg, other):
             del unit
     a, b = min(times[lg]), min(times[other])
     assert a < 1.12 * b, (a, b)
+
+
+@pytest.mark.parametrize("dtype,lg,batch,src_pack,dst_pack",
+                         [("float32", lg, b, s, d) for lg, b in ((15, 161), (15, 769), (16, 256))
+                          for s, d in ((1, 8), (8, 1), (2, 4))] +
+                         [("float64", 14, 97, s, d) for s, d in ((1, 4), (4, 1), (2, 4))])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_one_pass_in_place_between_small_packs(dtype, lg, batch, src_pack, dst_pack, inverse):
+    """In place with two different packs of up to one register: a workgroup has read its whole
+    transform before it writes, so the result is that of the out-of-place call bit for bit."""
+    import torch
+
+    import packed_amd as pa
+
+    n = 1 << lg
+    rt = torch.float32 if dtype == "float32" else torch.float64
+    src = torch.randn(batch * 2 * n, generator=torch.Generator("cuda").manual_seed(lg), device="cuda", dtype=rt)
+    dst = torch.zeros_like(src)
+    unit = pa.fft_unit(n, dtype=dtype)
+    for out in (dst, src):
+        unit.batch(out.data_ptr(), src.data_ptr(), batch, dst_pack, 2 * n, src_pack, 2 * n, inverse=inverse)
+    assert torch.equal(dst, src)
