@@ -1611,7 +1611,8 @@ int queue_build(pcx_queue_t q) {
             }
         }
     }
-    q->nitems = (int32_t)items.size();
+    q->nitems       = (int32_t)items.size();
+    int64_t tmp_min = 0; // one transform of the largest grouped size
     for (int lg = kMaxLog2; lg >= 1; --lg)
         for (int inv = 0; inv < 2; ++inv) {
             auto& b = bucket[lg * 2 + inv];
@@ -1628,8 +1629,12 @@ int queue_build(pcx_queue_t q) {
             else if (int e = pcx_plan_create((int64_t)1 << lg, 2048, PCX_ORDER_NORMAL, &g.plan))
                 return e;
             q->groups.push_back(g);
-            if (lg > kQueueMaxLog2)
-                q->tmp_bytes = std::max(q->tmp_bytes, std::min(g.count, g.plan->chunk) * 8 * g.plan->n);
+            if (lg > kQueueMaxLog2) {
+                // k_tile leaves less than a round of its sizes to the four-step
+                const int64_t most = g.plan->tw_tile ? g.plan->ncu : g.plan->chunk;
+                q->tmp_bytes       = std::max(q->tmp_bytes, std::min(g.count, most) * 8 * g.plan->n);
+                tmp_min            = std::max(tmp_min, 8 * g.plan->n);
+            }
         }
     hipStream_t setup = nullptr;
     hipError_t  he    = setup_stream(&setup);
@@ -1643,8 +1648,13 @@ int queue_build(pcx_queue_t q) {
     upload(&q->items, items);
     upload(&q->src_offs, qs);
     upload(&q->dst_offs, qd);
-    if (q->tmp_bytes > 0 && he == hipSuccess)
-        he = hipMalloc(&q->tmp, q->tmp_bytes);
+    if (q->tmp_bytes > 0 && he == hipSuccess) {
+        // on a full device less will do, down to one transform at a time
+        while ((he = hipMalloc(&q->tmp, q->tmp_bytes)) == hipErrorOutOfMemory && q->tmp_bytes > tmp_min) {
+            (void)hipGetLastError();
+            q->tmp_bytes = std::max(tmp_min, q->tmp_bytes / 2);
+        }
+    }
     if (q->tmp_bytes > 0 && he == hipSuccess)
         he = hipEventCreateWithFlags(&q->tmp_ev, hipEventDisableTiming);
     if (!items.empty() && he == hipSuccess) {

@@ -258,3 +258,20 @@ def test_tuning_file_of_the_earlier_queue(orc, pa, tmp_path):
     torch.cuda.synchronize()
     _check(orc, jobs, data, dst.cpu().numpy())
     assert cache.read_text() == text
+
+
+def test_queue_of_one_pass_transforms_needs_little_memory(pa):
+    """1500 transforms of 2^16 run one per CU without an intermediate but for the last round: the queue
+    holds one round's, not the 750 MiB of the whole list."""
+    import torch
+
+    n, count = 1 << 16, 1500
+    jobs = [(16, 0, k * 2 * n, k * 2 * n) for k in range(count)]
+    first = pa.fft_queue(jobs[:1])  # what the library itself holds
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    q = pa.fft_queue(jobs)
+    torch.cuda.synchronize()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert free - torch.cuda.mem_get_info()[0] < (cus + 64) * 8 * n
+    del first, q
