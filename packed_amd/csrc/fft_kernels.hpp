@@ -823,6 +823,15 @@ constexpr int row_lds_floats() {
     return RowShape<LA, G, T, PX>::DATA + TwTable<LA, T>::FLOATS + 2 * TW;
 }
 
+// Waves per SIMD of a row kernel.  Permuted stores from one exchange array need a few registers more
+// than the 64 of eight waves: 2^13 (512 threads) runs at six instead, without spills.  bit_reversed
+// forward, pack 8, us, eight / six: 64 transforms 10.9 / 10.4, 512 21.6 / 20.4, 4096 116 / 108, 32768
+// 819 / 788 (1024, one round of eight waves, 29.4 / 32.0).
+template<int ST, bool HALF>
+constexpr int row_waves(int threads, int lds_bytes) {
+    const int w = waves_per_simd(threads, lds_bytes);
+    return ST == ST_PERM && HALF && threads <= 512 && w > 6 ? 6 : w;
+}
 // Grid-stride over row groups: gridDim.x may be smaller than the number of groups.
 // The matrix-core variants keep the split operands in registers: they run at half the waves,
 // but at least two, so the register budget (256) never pushes accumulators into AGPRs.
@@ -830,8 +839,9 @@ constexpr int mfma_waves(int w, int prec) { return prec == PREC_FP32 ? w : (w > 
 
 template<int LA, int G, int LD, int ST, int TW, bool UNI, int ORD, int PREC = PREC_FP32, class T = float, int PX = 0>
 __global__ __launch_bounds__((G * Plan<LA, false, T, PX>::TA),
-                             mfma_waves(waves_per_simd(G * Plan<LA, false, T, PX>::TA,
-                                                       (int)sizeof(T) * row_lds_floats<LA, G, TW, T, PX>()),
+                             mfma_waves(row_waves<ST, Plan<LA, false, T, PX>::HALF>(
+                                            G * Plan<LA, false, T, PX>::TA,
+                                            (int)sizeof(T) * row_lds_floats<LA, G, TW, T, PX>()),
                                         PREC))
 void k_row(RowArgsT<T> p) {
     constexpr int NT = G * Plan<LA, false, T, PX>::TA;
