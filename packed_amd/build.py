@@ -19,7 +19,7 @@ OUT = os.path.join(HERE, "libpcx_gpu.so")
 
 # the slowest units first
 SOURCES = ["k_mfma_big.hip", "k_mfma_p1.hip", "k_mfma_p4.hip", "k_f64.hip", "k_shapes_alt.hip", "k_mfma.hip", "k_f64_alt.hip",
-           "k_shapes.hip", "k_shapes_small.hip", "k_single.hip", "k_xc.hip", "k_xc_block.hip", "k_tile.hip", "k_misc.hip", "pcx_gpu.hip"]
+           "k_shapes.hip", "k_shapes_small.hip", "k_single.hip", "k_xc.hip", "k_xc_block.hip", "k_tile.hip", "k_mixed.hip", "k_misc.hip", "pcx_gpu.hip"]
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",

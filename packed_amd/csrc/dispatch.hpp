@@ -285,6 +285,7 @@ void launch_tile(int lg, const TileArgs& a, int64_t grid, hipStream_t st);
 
 // ---- launchers of the remaining kernels (k_misc.hip)
 void launch_queue(const QueueArgs& a, int grid, hipStream_t st);
+void launch_mixed(const MixArgs& a, int grid, hipStream_t st); // k_mixed.hip
 void launch_vexpr(const VExprArgsT<float>& a, hipStream_t st);
 void launch_vexpr(const VExprArgsT<double>& a, hipStream_t st);
 

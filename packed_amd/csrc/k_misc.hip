@@ -1,97 +1,19 @@
 // k_misc.hip -- the persistent uneven-batch queue kernel (one launch for every transform of
 // 2^1 .. 2^14 points) and the vector-expression kernel.
 #include "dispatch.hpp"
+#include "queue_items.hpp"
 
 #include <algorithm>
 
 namespace pcxk {
 
-// LDS of the largest item (floats)
-template<int LA>
-constexpr int queue_single_lds() {
-    constexpr int PX = q_ppt(LA);
-    constexpr int G  = kQueueThreads / Plan<LA, false, float, PX>::TA;
-    return RowShape<LA, G, float, PX>::DATA + TwTable<LA>::FLOATS;
-}
-template<int... L>
-constexpr int queue_single_max(std::integer_sequence<int, L...>) {
-    int m = 0;
-    ((m = m > queue_single_lds<L + 1>() ? m : queue_single_lds<L + 1>()), ...);
-    return m;
-}
-constexpr int kQueueLds = queue_single_max(std::make_integer_sequence<int, kQueueMaxLog2>{});
+constexpr int kQueueLds = kQueueSingleLds<kQueueThreads>;
 static_assert(4 * kQueueLds <= 80 * 1024, "two workgroups fit one CU's LDS");
-
-// The queue kernel's LDS, at file scope: the item functions are compiled separately (each with
-// its own register budget) and address it directly as LDS.
-__shared__ float g_qlds[kQueueLds];
-
-// Values an item function receives arrive in VGPRs (function arguments); these make the
-// workgroup-uniform ones scalar again, so addresses and loop bounds stay in SGPRs.
-__device__ __forceinline__ int32_t uni(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ int64_t uni(int64_t v) {
-    const uint64_t u  = (uint64_t)v;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
-    return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-template<class T>
-__device__ __forceinline__ T* uni(T* p) {
-    return reinterpret_cast<T*>(uni((int64_t)reinterpret_cast<uintptr_t>(p)));
-}
-__device__ __forceinline__ QItem uni(const QItem& it) { return {uni(it.la), uni(it.inv), uni(it.first), uni(it.count)}; }
-
-// ---- single-pass item: `count` transforms of 2^LA points, one row of the workgroup each
-template<int LA>
-__device__ __noinline__ void queue_single(const QueueArgs& q, const QItem it_) {
-    float*      lds = g_qlds;
-    const QItem it  = uni(it_);
-    constexpr int PX = q_ppt(LA);
-    constexpr int TA = Plan<LA, false, float, PX>::TA;
-    constexpr int G  = kQueueThreads / TA;
-    static_assert(G * TA == kQueueThreads, "single-pass items fill the workgroup");
-    using S = RowShape<LA, G, float, PX>;
-    RowArgs p{};
-    p.src      = uni(q.src);
-    p.dst      = uni(q.dst);
-    p.src_offs = uni(q.src_offs) + it.first;
-    p.dst_offs = uni(q.dst_offs) + it.first;
-    p.src_size = (int64_t)1 << LA;
-    p.nrows    = it.count;
-    p.src_lp = p.dst_lp = LA;
-    p.rows_lg           = 0;
-    p.order             = 0;
-    p.conj_in = p.conj_out = it.inv;
-    p.scale                = (it.inv && uni(q.normalized)) ? 1.0f / (float)(1 << LA) : 1.0f;
-    p.twA                  = uni(q.tw) + ((1 << LA) - 2);
-    using LC               = LdsCarve<float, S::DATA, TwTable<LA>::FLOATS, 0>;
-    float* ltw             = lds + LC::TOFF;
-    float* lre             = lds + LC::DOFF;
-    TwTable<LA>::fill(ltw, p.twA, threadIdx.x, kQueueThreads);
-    __syncthreads();
-    row_group<LA, G, LD_CONTIG, ST_CONTIG, 0, (TA >= 64), 0, PREC_FP32, float, PX>(p, 0, lre, S::im(lre), ltw, nullptr);
-}
 
 __global__ __launch_bounds__(kQueueThreads, 4) void k_queue(QueueArgs q) {
     for (int it = (int)blockIdx.x; it < q.nitems; it += (int)gridDim.x) {
         const QItem w = q.items[it];
-        switch (w.la) {
-        case 1: queue_single<1>(q, w); break;
-        case 2: queue_single<2>(q, w); break;
-        case 3: queue_single<3>(q, w); break;
-        case 4: queue_single<4>(q, w); break;
-        case 5: queue_single<5>(q, w); break;
-        case 6: queue_single<6>(q, w); break;
-        case 7: queue_single<7>(q, w); break;
-        case 8: queue_single<8>(q, w); break;
-        case 9: queue_single<9>(q, w); break;
-        case 10: queue_single<10>(q, w); break;
-        case 11: queue_single<11>(q, w); break;
-        case 12: queue_single<12>(q, w); break;
-        case 13: queue_single<13>(q, w); break;
-        case 14: queue_single<14>(q, w); break;
-        default: break;
-        }
+        queue_single_any<kQueueThreads, kQueueLds>(q, w);
         __syncthreads(); // LDS is reused by the next item
     }
 }

@@ -9,9 +9,12 @@
 
 #include <array>
 #include <cstdio>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <mutex>
+#include <queue>
 #include <string>
 #include <utility>
 #include <vector>
@@ -1480,17 +1483,23 @@ struct pcx_queue_s {
     int                 normalized = 1;
     int64_t             njobs      = 0;
     double              flops = 0, bytes = 0;
-    // persistent part: transforms of 2^1 .. 2^14 points
+    // persistent part: transforms of 2^1 .. 2^14 points (k_queue), or of 2^1 .. 2^18 (k_mixed)
+    bool                mixed      = false;
+    int                 choice     = -1;      // of the two: as tuned, or -1 by queue_prefers_mixed
     int32_t             nitems     = 0;
     QItem*              items      = nullptr; // device
     int64_t*            src_offs   = nullptr; // per transform: items first, then the groups
     int64_t*            dst_offs   = nullptr;
     float2*             tw         = nullptr; // W_A for A = 2 .. 2^14
-    int                 grid       = 0;       // workgroups of the persistent launch
+    int                 grid       = 0;       // workgroups of k_queue
     int                 grid_cap   = 0;
-    // grouped part, largest size first: sizes above 2^14, and the classes the autotuner moved out of
-    // the persistent launch (grouped[log2n][inverse]); the groups run one after another through
-    // one four-step intermediate
+    float2*             ptw        = nullptr; // k_mixed: pass tables, the item counter
+    int32_t             ptw_off[kMixMaxLog2 + 1] = {};
+    uint32_t*           counter    = nullptr;
+    int64_t             mix_floats = 0;       // of a workgroup's intermediate
+    // grouped part, largest size first: the sizes above the persistent part's, and the classes the autotuner moved out of
+    // k_queue (grouped[log2n][inverse]); the groups run one after another through one four-step
+    // intermediate (k_mixed's workgroups have theirs in it, too)
     std::vector<QGroup> groups;
     void*               tmp        = nullptr;
     int64_t             tmp_bytes  = 0;
@@ -1536,16 +1545,22 @@ int queue_on_tmp(pcx_queue_t q, hipStream_t st, F&& fn) {
 }
 
 int queue_run(pcx_queue_t q, float* dst, const float* src, hipStream_t st) {
-    if (q->nitems > 0) {
-        QueueArgs a{};
-        a.src = src, a.dst = dst;
-        a.src_offs = q->src_offs, a.dst_offs = q->dst_offs;
-        a.items = q->items, a.nitems = q->nitems, a.normalized = q->normalized;
-        a.tw = q->tw;
+    QueueArgs a{};
+    a.src = src, a.dst = dst;
+    a.src_offs = q->src_offs, a.dst_offs = q->dst_offs;
+    a.items = q->items, a.nitems = q->nitems, a.normalized = q->normalized;
+    a.tw = q->tw;
+    if (q->nitems > 0 && !q->mixed) {
         launch_queue(a, std::min<int>(q->grid, q->nitems), st);
         HIPCHK(hipGetLastError());
     }
     return queue_on_tmp(q, st, [&] {
+        if (q->mixed) {
+            MixArgs m{a, (float*)q->tmp, q->mix_floats, q->counter, q->ptw, {}};
+            std::copy(std::begin(q->ptw_off), std::end(q->ptw_off), m.ptw_off);
+            launch_mixed(m, std::min<int>(q->grid_cap / 2, q->nitems), st);
+            HIPCHK(hipGetLastError());
+        }
         for (const auto& g : q->groups)
             if (int e = queue_run_group(q, g, dst, src, st))
                 return e;
@@ -1569,7 +1584,10 @@ void queue_release(pcx_queue_t q) {
     (void)hipFree(q->src_offs);
     (void)hipFree(q->dst_offs);
     (void)hipFree(q->tw);
+    (void)hipFree(q->ptw);
+    (void)hipFree(q->counter);
     (void)hipFree(q->tmp);
+    q->ptw = nullptr, q->counter = nullptr, q->mixed = false, q->mix_floats = 0;
     q->items = nullptr, q->src_offs = q->dst_offs = nullptr, q->tw = nullptr, q->nitems = 0;
     q->tmp = nullptr, q->tmp_bytes = 0;
     for (auto& g : q->groups)
@@ -1583,8 +1601,67 @@ void queue_free(pcx_queue_t q) {
     delete q;
 }
 
-// Builds the persistent items (every class up to 2^14 not marked grouped) and the grouped launches
-// (the rest), both largest first, from the job list.
+using QueueCounts = std::array<std::array<int64_t, 2>, kMaxLog2 + 1>; // transforms by size and direction
+
+// Whether the sizes up to 2^18 of a list run faster as one launch of workgroups that take whole
+// transforms (k_mixed) than as k_queue and a full-chip launch per class, from the times that these take
+// on `ncu` CUs, us:
+//   k_mixed   0.97 the longest workgroup's load + 0.8 the mean one + 0.46 as much again, up to half of
+//             the longest transform (the chip is shared from the first transform on); a load counts
+//             a transform's time on an otherwise empty chip;
+//   per class 12.5 and a time per transform, or rounds of one transform per CU (k_tile, and one-array
+//             passes of 2^15); 15 and 6 per 10^6 points for k_queue.
+// Over 420 lists (16 .. 2000 jobs, smallest 2^4 .. 2^18, largest 2^15 .. 2^19, either direction or both)
+// the choice is 0.4 % from the faster of the two on average and 6 % at worst.  Launches per class alone:
+// 1.9 % on average and 21 % at worst (more than 3 % for 71 lists); k_mixed alone 41 %, and 6.2 times.
+bool queue_prefers_mixed(const QueueCounts& n, int ncu) {
+    constexpr double kAlone[4][2] = {{35, 45}, {63, 68}, {112, 121}, {246, 263}}; // 2^15 .. 2^18
+    constexpr double kEach[4]     = {0.166, 0.389, 0.863, 1.863};
+    const double     scale        = 256.0 / ncu;
+    double split = 0, total = 0, longest = 0, small = 0; // small: points up to 2^14
+    std::vector<double> load(ncu, 0.0);
+    std::priority_queue<double, std::vector<double>, std::greater<double>> least(std::greater<double>(), std::move(load));
+    auto take = [&](double us, int64_t count) {
+        for (int64_t k = 0; k < count; ++k) {
+            const double l = least.top() + us;
+            least.pop();
+            least.push(l);
+            longest = std::max(longest, l);
+        }
+        total += us * (double)count;
+    };
+    double one   = 0; // the longest transform
+    int    sizes = 0;
+    for (int lg = kMixMaxLog2; lg > kQueueMaxLog2; --lg) {
+        sizes += n[lg][0] + n[lg][1] > 0;
+        for (int inv = 1; inv >= 0; --inv) {
+            const int     k     = lg - kQueueMaxLog2 - 1;
+            const int64_t count = n[lg][inv];
+            if (count == 0)
+                continue;
+            take(kAlone[k][inv], count);
+            one                = std::max(one, kAlone[k][inv]);
+            const int64_t last = count % ncu, tiles = lg != 16 ? 0 : 10 * last > 7 * ncu ? count : count - last;
+            if (lg == 15 && count >= kOnePassBatch)
+                split += 28.6 * (double)((count + ncu - 1) / ncu) + 0.06 * scale * (double)count;
+            else if (count > tiles)
+                split += 12.5 + kEach[k] * scale * (double)(count - tiles);
+            split += 71 * (double)((tiles + ncu - 1) / ncu);
+        }
+    }
+    if (sizes < 2) // nothing to mix: launches per class are faster
+        return false;
+    for (int lg = 1; lg <= kQueueMaxLog2; ++lg)
+        small += (double)((n[lg][0] + n[lg][1]) << lg);
+    if (small > 0)
+        split += 15 + 6e-6 * scale * small;
+    take(9, (int64_t)std::ceil(small / 16384));
+    const double mean = total / ncu;
+    return 1.02 * (0.97 * longest + 0.8 * mean + 0.46 * std::min(mean, one / 2)) < split;
+}
+
+// Builds the persistent items (every class up to 2^18 with k_mixed, else up to 2^14, not marked
+// grouped) and the grouped launches (the rest), both largest first, from the job list.
 int queue_build(pcx_queue_t q) {
     const pcx_job* jobs  = q->jobs.data();
     const int64_t  njobs = (int64_t)q->jobs.size();
@@ -1597,10 +1674,27 @@ int queue_build(pcx_queue_t q) {
         qs.push_back(jobs[job].src_offset);
         qd.push_back(jobs[job].dst_offset);
     };
-    for (int lg = kQueueMaxLog2; lg >= 1; --lg) {
-        const int per = std::max(1, kQueueThreads / (lg >= 4 ? (1 << lg) / 16 : 1));
+    const int   ncu = q->grid_cap / 2;
+    QueueCounts n{};
+    for (int lg = 1; lg <= kMaxLog2; ++lg)
+        n[lg] = {(int64_t)bucket[2 * lg].size(), (int64_t)bucket[2 * lg + 1].size()};
+    int four = 0; // the largest four-step size of k_mixed
+    for (int lg = kQueueMaxLog2 + 1; lg <= kMixMaxLog2; ++lg)
+        four = n[lg][0] + n[lg][1] > 0 ? lg : four;
+    // by estimate only for vectors on whole 128-byte lines: k_mixed loses a quarter of its rate on others,
+    // launches per class 3 - 7 % (1000 of 2^12 .. 2^18: 567 -> 747 us, 654 -> 691)
+    bool lines = true;
+    for (const pcx_job& j : q->jobs)
+        if (j.log2n > kQueueMaxLog2)
+            lines = lines && ((j.src_offset | j.dst_offset) & 31) == 0;
+    q->mixed          = four > 0 && (q->choice < 0 ? lines && queue_prefers_mixed(n, ncu) : q->choice == 1);
+    const int top     = q->mixed ? kMixMaxLog2 : kQueueMaxLog2;
+    const int threads = q->mixed ? kMixThreads : kQueueThreads;
+    auto      persistent = [&](int lg, int inv) { return lg <= top && (lg > kQueueMaxLog2 || !q->grouped[lg][inv]); };
+    for (int lg = top; lg >= 1; --lg) {
+        const int per = std::max(1, threads / (lg >= 4 ? (1 << lg) / 16 : 1));
         for (int inv = 0; inv < 2; ++inv) {
-            if (q->grouped[lg][inv])
+            if (!persistent(lg, inv))
                 continue;
             auto& b = bucket[lg * 2 + inv];
             for (size_t k = 0; k < b.size(); k += per) {
@@ -1616,7 +1710,7 @@ int queue_build(pcx_queue_t q) {
     for (int lg = kMaxLog2; lg >= 1; --lg)
         for (int inv = 0; inv < 2; ++inv) {
             auto& b = bucket[lg * 2 + inv];
-            if (b.empty() || (lg <= kQueueMaxLog2 && !q->grouped[lg][inv]))
+            if (b.empty() || persistent(lg, inv))
                 continue;
             QGroup g;
             g.lg = lg, g.inv = inv, g.count = (int64_t)b.size(), g.first = (int64_t)qs.size();
@@ -1648,11 +1742,22 @@ int queue_build(pcx_queue_t q) {
     upload(&q->items, items);
     upload(&q->src_offs, qs);
     upload(&q->dst_offs, qd);
+    if (q->mixed) { // every workgroup its own intermediate of the largest size
+        q->mix_floats = (int64_t)2 << four;
+        q->tmp_bytes  = std::max<int64_t>(q->tmp_bytes, 4 * q->mix_floats * std::min<int64_t>(ncu, q->nitems));
+        tmp_min       = std::max(tmp_min, q->tmp_bytes);
+    }
     if (q->tmp_bytes > 0 && he == hipSuccess) {
         // on a full device less will do, down to one transform at a time
         while ((he = hipMalloc(&q->tmp, q->tmp_bytes)) == hipErrorOutOfMemory && q->tmp_bytes > tmp_min) {
             (void)hipGetLastError();
             q->tmp_bytes = std::max(tmp_min, q->tmp_bytes / 2);
+        }
+        if (he == hipErrorOutOfMemory && q->mixed) { // launches per class need less
+            (void)hipGetLastError();
+            queue_release(q);
+            q->choice = 0;
+            return queue_build(q);
         }
     }
     if (q->tmp_bytes > 0 && he == hipSuccess)
@@ -1661,6 +1766,21 @@ int queue_build(pcx_queue_t q) {
         he = hipMalloc(&q->tw, sizeof(float2) * ((1 << (kQueueMaxLog2 + 1)) - 2));
         for (int lg = 1; lg <= kQueueMaxLog2 && he == hipSuccess; ++lg)
             he = gen_twiddles(q->tw + ((1 << lg) - 2), (int64_t)1 << lg, 1, (int64_t)1 << lg, setup);
+        if (he == hipSuccess && q->mixed) {
+            // pass tables W_N^e = lo[e mod 2^ls] * hi[e >> ls] of every four-step size
+            int32_t at = 0;
+            for (int lg = kQueueMaxLog2 + 1; lg <= four; ++lg)
+                q->ptw_off[lg] = at, at += pass_tw_entries(lg);
+            he = hipMalloc(&q->ptw, sizeof(float2) * at);
+            for (int lg = kQueueMaxLog2 + 1; lg <= four && he == hipSuccess; ++lg) {
+                const int64_t nl = (int64_t)1 << (lg + 1) / 2, size = (int64_t)1 << lg;
+                he = gen_twiddles(q->ptw + q->ptw_off[lg], size, 1, nl, setup);
+                if (he == hipSuccess)
+                    he = gen_twiddles(q->ptw + q->ptw_off[lg] + nl, size, nl, size / nl, setup);
+            }
+            if (he == hipSuccess)
+                he = hipMalloc(&q->counter, sizeof(uint32_t));
+        }
         if (he == hipSuccess)
             he = hipStreamSynchronize(setup);
     }
@@ -1815,8 +1935,8 @@ float time_ms(hipStream_t st, F&& fn, int reps = 3) {
 
 } // namespace
 
-// Autotuner: workgroups of the persistent launch, then per grouped size the four-step shape and
-// grid caps.  Winners are written to cache_path (one "key value..." line each) and read back
+// Autotuner: k_mixed or launches per class, workgroups of k_queue, then per grouped size the four-step
+// shape and grid caps.  Winners are written to cache_path (one "key value..." line each) and read back
 // from it when present.
 extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, void* stream, const char* cache_path) {
     if (!q)
@@ -1842,17 +1962,22 @@ extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, v
             char key[32];
             int  a = 0, b = 0, c = 0, d = 0, e = 0;
             long long gc = 0, gr = 0;
-            // the split between the persistent launch and grouped launches comes first
+            // the split between the persistent launch and grouped launches comes first (a file without
+            // a "mixed" line leaves that choice as it is)
             bool mask[kQueueMaxLog2 + 1][2] = {};
+            int  choice = q->choice;
             long pos = std::ftell(f);
             while (std::fscanf(f, "%31s", key) == 1) {
                 if (!std::strcmp(key, "grouped") && std::fscanf(f, "%d %d", &a, &b) == 2 && a >= 1 && a <= kQueueMaxLog2 &&
                     (b == 0 || b == 1))
                     mask[a][b] = true;
+                else if (!std::strcmp(key, "mixed") && std::fscanf(f, "%d", &a) == 1 && (a == 0 || a == 1))
+                    choice = a;
             }
             std::fseek(f, pos, SEEK_SET);
-            if (std::memcmp(mask, q->grouped, sizeof(mask)) != 0) {
+            if (std::memcmp(mask, q->grouped, sizeof(mask)) != 0 || choice != q->choice) {
                 std::memcpy(q->grouped, mask, sizeof(mask));
+                q->choice = choice;
                 queue_release(q);
                 if (int err = queue_build(q)) {
                     std::fclose(f);
@@ -1861,6 +1986,8 @@ extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, v
             }
             while (std::fscanf(f, "%31s", key) == 1) {
                 if (!std::strcmp(key, "grouped") && std::fscanf(f, "%d %d", &a, &b) == 2) {
+                    continue;
+                } else if (!std::strcmp(key, "mixed") && std::fscanf(f, "%d", &a) == 1) {
                     continue;
                 } else if (!std::strcmp(key, "queue_grid") && std::fscanf(f, "%d", &a) == 1) {
                     q->grid = std::max(1, std::min(a, q->grid_cap));
@@ -1888,7 +2015,31 @@ extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, v
             return PCX_SUCCESS;
         }
     }
-    if (q->nitems > 0) {
+    auto whole   = [&] { return queue_run(q, dst, src, st); };
+    auto rebuild = [&]() -> int {
+        queue_release(q);
+        return queue_build(q);
+    };
+    // one launch over the sizes up to 2^18, or launches per class
+    bool four = false;
+    for (const auto& j : q->jobs)
+        four = four || (j.log2n > kQueueMaxLog2 && j.log2n <= kMixMaxLog2);
+    if (four) {
+        std::memset(q->grouped, 0, sizeof(q->grouped));
+        float ms[2];
+        for (int c = 1; c >= 0; --c) {
+            q->choice = c;
+            if (int e = rebuild())
+                return e;
+            ms[c] = q->mixed == (c == 1) ? time_ms(st, whole) : 1e30f; // (no room for k_mixed)
+        }
+        if (ms[1] < ms[0]) {
+            q->choice = 1;
+            if (int e = rebuild())
+                return e;
+        }
+    }
+    if (q->nitems > 0 && !q->mixed) {
         float best = 1e30f;
         int   bg   = q->grid;
         for (int grid : {q->grid_cap / 2, (3 * q->grid_cap) / 4, q->grid_cap}) {
@@ -1907,18 +2058,12 @@ extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, v
         }
         q->grid = bg;
     }
-    // the sizes of the persistent launch move out to grouped launches when that makes the whole pass
-    // faster
-    {
+    // the sizes of k_queue move out to grouped launches when that makes the whole pass faster
+    if (!q->mixed) {
         bool present[kQueueMaxLog2 + 1] = {}, any = false;
         for (const auto& j : q->jobs)
             if (j.log2n <= kQueueMaxLog2)
                 present[j.log2n] = any = true;
-        auto whole   = [&] { return queue_run(q, dst, src, st); };
-        auto rebuild = [&]() -> int {
-            queue_release(q);
-            return queue_build(q);
-        };
         if (any) {
             const float best = time_ms(st, whole);
             for (int lg = 1; lg <= kQueueMaxLog2; ++lg)
@@ -1975,6 +2120,8 @@ extern "C" int pcx_queue_autotune(pcx_queue_t q, float* dst, const float* src, v
                 if (g.plan->two_pass)
                     std::fprintf(f, "group %d %d %d %d %d %lld %lld\n", g.lg, g.inv, g.plan->shape->n2, g.plan->shape->g,
                                  g.plan->shape->c, (long long)g.plan->grid_col, (long long)g.plan->grid_row);
+            if (four)
+                std::fprintf(f, "mixed %d\n", q->mixed ? 1 : 0);
             std::fclose(f);
         }
     }

@@ -275,3 +275,82 @@ def test_queue_of_one_pass_transforms_needs_little_memory(pa):
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     assert free - torch.cuda.mem_get_info()[0] < (cus + 64) * 8 * n
     del first, q
+
+
+def _many(seed, jobs, low, high):
+    rng = np.random.default_rng(seed)
+    return _jobs(rng, [int(v) for v in rng.integers(low, high + 1, jobs)])
+
+
+@pytest.mark.parametrize("normalized", [True, False])
+@pytest.mark.parametrize("mixed", [0, 1])
+def test_one_launch_over_mixed_sizes_or_launches_per_class(orc, pa, tmp_path, mixed, normalized):
+    """Both forms of the sizes up to 2^18 (named by a tuning file), of every size from 2 on: eager, in
+    place, and replayed with eager work between the replays; larger sizes run beside either."""
+    import torch
+
+    rng = np.random.default_rng(11)
+    sizes = list(range(1, 20)) * 2 + [1, 3, 14, 15, 15, 15, 16, 16, 17, 18, 18] + [int(v) for v in rng.integers(5, 17, 60)]
+    rng.shuffle(sizes)
+    jobs, total = _jobs(rng, sizes)
+    buf, data = _fill(orc, jobs, total)
+    src = torch.from_numpy(buf).cuda()
+    dst = torch.zeros_like(src)
+    cache = tmp_path / "tune.txt"
+    cache.write_text(f"queue_grid 512\nmixed {mixed}\n")
+    q = pa.fft_queue(jobs, normalized=normalized)
+    q.autotune(dst.data_ptr(), src.data_ptr(), str(cache))
+    for rep in range(2):
+        dst.zero_()
+        q.exec(dst.data_ptr(), src.data_ptr())
+        torch.cuda.synchronize()
+        _check(orc, jobs, data, dst.cpu().numpy(), normalized)
+    want = dst.clone()
+    s = torch.cuda.Stream()
+    q.capture(dst.data_ptr(), src.data_ptr(), s)
+    for rep in range(3):
+        dst.zero_()
+        torch.cuda.synchronize()
+        q.launch(s)
+        s.synchronize()
+        assert torch.equal(dst, want)
+        torch.randn(1 << 20, device="cuda").mul_(2)
+        torch.cuda.synchronize()
+    q.exec(src.data_ptr(), src.data_ptr())
+    torch.cuda.synchronize()
+    for lg, _, _, do in jobs:  # (the gaps between the vectors are src's own)
+        assert torch.equal(src[do:do + (2 << lg)], want[do:do + (2 << lg)])
+
+
+@pytest.mark.parametrize("lines", [False, True])
+@pytest.mark.parametrize("jobs,low,high", [(1400, 7, 16), (1000, 10, 17), (1000, 12, 18), (50, 4, 18), (400, 16, 16)])
+def test_the_faster_of_the_two_forms_is_chosen(pa, tmp_path, jobs, low, high, lines):
+    """Where the forms differ by a fifth and more: many classes of moderate count run as one launch, few
+    transforms or one large class as launches per class.  The choice is within 10 % of the faster."""
+    import torch
+
+    todo, total = _many(jobs + high, jobs, low, high)
+    if lines:  # every vector on whole 128-byte lines
+        todo = [(lg, inv, (so + 31) // 32 * 32 + 32 * k, (do + 31) // 32 * 32 + 32 * k)
+                for k, (lg, inv, so, do) in enumerate(todo)]
+        total += 32 * jobs + 32
+    src = torch.randn(total, device="cuda")
+    dst = torch.zeros_like(src)
+    times = []
+    for mixed in (None, 0, 1):
+        q = pa.fft_queue(todo)
+        if mixed is not None:
+            cache = tmp_path / f"{mixed}.txt"
+            cache.write_text(f"queue_grid 512\nmixed {mixed}\n")
+            q.autotune(dst.data_ptr(), src.data_ptr(), str(cache))
+        best = float("inf")
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(3):
+                q.exec(dst.data_ptr(), src.data_ptr())
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        times.append(best)
+    assert times[0] < 1.1 * min(times[1:]), times
