@@ -495,9 +495,9 @@ def run_config3(args):
 
 def run_config4(args):
     """10,000 FP32 C2C transforms, sizes 2^6..2^20 drawn log-uniform (seeded), complex normal
-    inputs, mixed directions: the work queue (every transform in one persistent launch, eager and
-    as a hipGraph; then autotuned, where the tuner may move size classes to grouped launches after
-    the persistent one) vs one launch per size class and one launch per transform."""
+    inputs, mixed directions: the work queue (one persistent launch and full-chip launches per larger
+    size, or one launch over the sizes up to 2^18; eager and as a hipGraph, then autotuned) vs one
+    launch per size class and one launch per transform."""
     import numpy as np
     import torch
 
@@ -530,7 +530,7 @@ def run_config4(args):
         return {"ms": round(ms, 3), "gflops": round(flops / (ms * 1e-3) / 1e9, 1),
                 "gbps": round(algo_bytes / (ms * 1e-3) / 1e9, 1)}
 
-    # the default queue: every transform in one persistent launch
+    # the default queue, eager and captured
     res["queue_eager"] = rate(time_steps(lambda: q.exec(dst.data_ptr(), src.data_ptr()), 5, 1))
     s1 = torch.cuda.Stream()
     q.capture(dst.data_ptr(), src.data_ptr(), s1)
