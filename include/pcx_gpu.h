@@ -219,11 +219,11 @@ int     pcx_fxcorr_exec_batch_ws(pcx_fxcorr_t xc, float* dst, int64_t dst_pack, 
  * direction, one after another through one four-step intermediate of the queue (that of the class
  * that needs most, at most 2 GiB; less on a full device).  Where many classes of moderate count meet,
  * all sizes up to 2^18 run in one launch instead, each transform in one workgroup (the queue then
- * holds an intermediate of the largest such size per CU).  Passes on different streams, pcx_queue_exec and
- * pcx_queue_launch alike, wait for one another at the intermediate (replays of a capture that the
- * caller makes of pcx_queue_exec do not).  pcx_queue_capture records the whole pass into a hipGraph
- * for fixed (dst, src); pcx_queue_autotune times the launch shapes on the caller's data and keeps
- * the fastest (optionally persisted in a cache file). */
+ * holds an intermediate of the largest such size per CU).  Passes on different streams,
+ * pcx_queue_exec and pcx_queue_launch alike, wait for one another at the intermediate (replays of a
+ * capture that the caller makes of pcx_queue_exec do not).  pcx_queue_capture records the whole pass
+ * into a hipGraph for fixed (dst, src); pcx_queue_autotune times the launch shapes on the caller's
+ * data and keeps the fastest (optionally persisted in a cache file). */
 typedef struct {
     int64_t log2n;      /* transform size 2^log2n, 1 <= log2n <= 24 */
     int32_t inverse;    /* 0 forward, 1 inverse */

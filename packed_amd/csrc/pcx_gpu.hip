@@ -8,8 +8,8 @@
 #include <hip/hip_runtime.h>
 
 #include <array>
-#include <cstdio>
 #include <cmath>
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
@@ -1497,9 +1497,9 @@ struct pcx_queue_s {
     int32_t             ptw_off[kMixMaxLog2 + 1] = {};
     uint32_t*           counter    = nullptr;
     int64_t             mix_floats = 0;       // of a workgroup's intermediate
-    // grouped part, largest size first: the sizes above the persistent part's, and the classes the autotuner moved out of
-    // k_queue (grouped[log2n][inverse]); the groups run one after another through one four-step
-    // intermediate (k_mixed's workgroups have theirs in it, too)
+    // grouped part, largest size first: the sizes above the persistent part's, and the classes the
+    // autotuner moved out of k_queue (grouped[log2n][inverse]); the groups run one after another
+    // through one four-step intermediate (k_mixed's workgroups have theirs in it, too)
     std::vector<QGroup> groups;
     void*               tmp        = nullptr;
     int64_t             tmp_bytes  = 0;
